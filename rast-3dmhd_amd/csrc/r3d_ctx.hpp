@@ -10,26 +10,11 @@
 #include <vector>
 
 #include "r3d_aux.hpp"
+#include "r3d_plan.hpp"
 #include "r3d_hip.h"
 
 namespace r3d {
 
-constexpr int TILE_Y = 9;  // the larger hydro stage tile (waves 1..9 compute fluxes)
-// Hydro tile rows for a grid npy cells high: 8 (11 waves; the 8 flux waves
-// sit two per SIMD, which measures faster than 9 rows with three flux waves on
-// one SIMD) unless 9 leaves fewer rows of the last tile idle.
-inline int hydro_tile_rows(int npy) {
-    const int w9 = (npy + 8) / 9 * 9 - npy, w8 = (npy + 7) / 8 * 8 - npy;
-    return w9 < w8 ? TILE_Y : 8;
-}
-// MHD tiles: 8 waves per workgroup (two per SIMD), so that the larger MHD
-// working set gets 256 VGPRs per lane instead of 168: 12 rows of 32 columns
-// (six flux waves of two rows each), or 5 rows of 64 columns (five flux
-// waves, the first tiling; 4% slower at 252x252x512, kept as an override)
-constexpr int TILE_Y_MAG = 12, TILE_W_MAG = 32;
-constexpr int TILE_Y_MAG64 = 5;
-// Columns of a stage tile of ty rows.
-inline int tile_width(bool lmag, int ty) { return lmag && ty == TILE_Y_MAG ? TILE_W_MAG : 64; }
 constexpr int DT_BLOCKS = 1024;
 
 // Set the calling thread's error message and return code.
@@ -79,7 +64,7 @@ struct r3d_hip_ctx {
     bool metrics_set = false;
     bool next_valid = false;  // scal->dt_next holds the dt of the current state
     std::vector<char> uploaded;
-    int ty = r3d::TILE_Y, tw = 64, ntx = 0, nty = 0, nkc = 0, kc = 0, nblocks = 0, grid = 0, nbb = 0;
+    int ty = r3d::TILE_Y, tw = 64, ntx = 0, nty = 0, nkc = 0, kc = 0, kq = 0, krem = 0, nblocks = 0, grid = 0, nbb = 0;
     unsigned long long bytes = 0;
     bool timing = false;
     long launches[4] = {0, 0, 0, 0};

@@ -123,7 +123,9 @@ struct StageArgs {
     int zmode;         // 0: Z' = mix (X' + zeta dt F); 1: Z' = X (save_state); 2: no Z write
     int want_dt;       // stage 3 of a full step: emit dt partials of X'
     int screen;        // stage 3: screen cells against the previous extrema (DevScal)
-    int ntx, nty, nkc, kc, nblocks;
+    // z chunk kz of a column tile has kq planes, the first krem chunks one more
+    // (the last one ends at npz)
+    int ntx, nty, nkc, kq, krem, nblocks;
 };
 
 // Number of dt partial slots per block: max of (ogamma uu/tt), min of the

@@ -53,7 +53,8 @@ __device__ __forceinline__ StageArgs member_args(const EnsMember& e, int cur, in
     a.ntx = e.ntx;
     a.nty = e.nty;
     a.nkc = e.nkc;
-    a.kc = e.kc;
+    a.kq = e.kc;
+    a.krem = 0;
     a.nblocks = e.nblocks;
     return a;
 }

@@ -498,7 +498,8 @@ StageArgs stage_args(r3d_hip_ctx* c, int stage, int zmode, int want_dt) {
     a.ntx = c->ntx;
     a.nty = c->nty;
     a.nkc = c->nkc;
-    a.kc = c->kc;
+    a.kq = c->kq;
+    a.krem = c->krem;
     a.nblocks = c->nblocks;
     return a;
 }
@@ -814,6 +815,8 @@ int r3d_hip_create(const r3d_hip_cfg* cfg, r3d_hip_ctx** out) {
         f.zchunk != 128)
         return set_err(R3D_EINVAL, "zchunk %d: one of 8, 16, 32, 64, 128", f.zchunk);
     HIPCHK(hipSetDevice(f.device));
+    int cus = 0;
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, f.device));
 
     auto* c = new r3d_hip_ctx();
     c->cfg = f;
@@ -831,21 +834,16 @@ int r3d_hip_create(const r3d_hip_cfg* cfg, r3d_hip_ctx** out) {
     c->uploaded.assign((size_t)f.npey * f.npez, 0);
     fill_consts(c);
 
-    // stage tiling: 64 x ty columns, z chunks sized for >= ~8 blocks per CU
-    c->ty = f.lmag ? TILE_Y_MAG : feature ? 8 : hydro_tile_rows(f.npy);
-    if (f.tile_rows) c->ty = f.tile_rows;
-    c->tw = tile_width(f.lmag != 0, c->ty);
-    c->ntx = (f.npx + c->tw - 1) / c->tw;
-    c->nty = (f.npy + c->ty - 1) / c->ty;
-    c->kc = 8;
-    for (int kc : {128, 64, 32, 16, 8}) {
-        if ((long)c->ntx * c->nty * ((f.npz + kc - 1) / kc) >= 2048) {
-            c->kc = kc;
-            break;
-        }
-    }
-    if (f.zchunk) c->kc = f.zchunk;
-    c->nkc = (f.npz + c->kc - 1) / c->kc;
+    const StagePlan pl = plan_stage(f.npx, f.npy, f.npz, f.lmag != 0, feature, f.tile_rows,
+                                    f.zchunk, cus);
+    c->ty = pl.ty;
+    c->tw = pl.tw;
+    c->ntx = pl.ntx;
+    c->nty = pl.nty;
+    c->kc = pl.kc;
+    c->kq = pl.kq;
+    c->krem = pl.krem;
+    c->nkc = pl.nkc;
     c->nblocks = c->ntx * c->nty * c->nkc;
     c->grid = (c->nblocks + 7) / 8 * 8;
     c->nbb = ((f.npx + 2) * (f.npy + 2) + BOUND_THREADS - 1) / BOUND_THREADS;
