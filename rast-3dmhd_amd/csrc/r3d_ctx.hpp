@@ -34,6 +34,7 @@ struct r3d_hip_ctx {
     r3d_hip_cfg cfg;
     r3d::Geo g;
     int nf = 5;
+    int cus = 0;  // compute units of the device
     int nx = 0, ny = 0, nz = 0, nry = 0, nrz = 0;
     hipStream_t stream = nullptr;
     double* xs[2][r3d::NXF] = {};  // X ping-pong; xs[cur] is the current state
@@ -45,9 +46,8 @@ struct r3d_hip_ctx {
     // per-plane extras (density diffusion, flux relaxation): per-(plane, y
     // rank) partial means, then ROM, the two diffusion coefficient rows, the
     // ID=2 wall profile, TTM, FCONM and RLAX*TFAC*CORRECT, (npz+2) each, and
-    // the relaxation state TFAC, TTM_MAX
+    // the relaxation state TFAC, TTM_MAX and the z ranks' offsets of CORRECT
     double* den_buf = nullptr;
-    double* ww2_buf = nullptr;  // flux relaxation: the convective flux WW2, one field
     double* stage_buf = nullptr;
     double* gstage = nullptr;  // one global field, (npx+2)(npy+2)(npz+2), allocated on first use
     // asynchronous snapshot (r3d_hip_snapshot_begin): X and Z as dense global

@@ -140,66 +140,146 @@ __global__ __launch_bounds__(DEN_THREADS) void k_den_mirror(const Geo g, double*
     ro[g.at(i, j, g.npz + 1)] = ro[g.at(si, sj, g.npz - 1)];
 }
 
-// Horizontal mean, first half (src/communicate.cpp:193-199): thread
-// (K, q) sums y rank q's interior rows of global plane K, j outer and i
-// inner, in one sequential chain, and divides by npx*npy.  The loads of a
-// row run ahead of the additions, which keep their order.  There are only
-// (npz+2)*npey chains, so blocks are one wave each and spread over every CU:
-// the speed is then the number of loads each lane keeps in flight.
-constexpr int DEN_PARTIAL_THREADS = 64;
-__device__ __forceinline__ void hmean_partial_chain(const Geo& g, const double* ro, double* part,
-                                                    int npey, double cnt) {
-    const int t = blockIdx.x * DEN_PARTIAL_THREADS + threadIdx.x;
-    if (t >= (g.npz + 2) * npey) return;
-    const int K = t / npey, q = t % npey, nry = g.npy / npey;
-    // 16-byte loads (rows start on 128-byte boundaries), 32 in flight
-    constexpr int U2 = 32, U = 16;
-    double sum = 0.0;
-    for (int j = q * nry + 1; j <= (q + 1) * nry; ++j) {
-        const double* row = ro + g.at(1, j, K);
-        int i = 0;
-        for (; i + 2 * U2 <= g.npx; i += 2 * U2) {
-            double2 v[U2];
+// Horizontal mean, first half (src/communicate.cpp:193-199): chain (K, q)
+// sums y rank q's interior rows of global plane K, j outer and i inner, in
+// one sequential chain, and divides by npx*npy.
+//
+// A chain's length in dependent additions bounds it (252 x 63 rows: 15876 of
+// them, some 4 ns each with their LDS reads), so a lane does nothing else.
+// One wave of the block sums its NCH chains, a lane each, out of LDS; the
+// three others keep the next 192 values of every chain coming, whole lines
+// at a time, and write them to LDS a segment later.  Rows of 194
+// doubles put the lanes' 16-byte LDS reads on different banks.  Four waves,
+// one per SIMD, so that three blocks share a CU at this register count (with
+// five, the fifth falls on the first SIMD and one block fills the CU), each
+// with its summing wave on another SIMD.  At 252x252x512 / npey 4, 2056
+// chains: 95 us; one lane loading its own chain (64 chains to a wave, 32
+// 16-byte loads in flight, each its own cache line): 570 us.
+// Chains per block: the fewest that spread them over the chip; 8 at most, 4
+// with WW2, whose loads (1.3 GB) bound it there: 275 us with 4 chains, 331 with
+// 8, against 293 + 574 us for a kernel that wrote WW2 out and the sum of it.
+//
+// WW2: the value summed is the convective flux
+// WW2 = -RW*(2.5*(TT-TTM(K)) + 0.5*(UU*UU+VV*VV+WW*WW)), UU = RU*(1/RO)
+// (golden/fortran/3dmhdsub.f:1656-1666), formed by the loading waves;
+// otherwise field x.q[f].
+// One chain a block (fewer chains than CUs) takes segments of 704 values, and
+// the block the CU: its per-segment barrier and first LDS reads then weigh less
+// (504x504x24 with one y rank, 26 chains of 254016:
+// a density diffusion step takes 4.5 ms, 5.1 with 192).
+constexpr int hm_seg(int nch) { return nch == 1 ? 704 : 192; }
+template <int NCH, bool WW2>
+__global__ __launch_bounds__(hm_seg(NCH) + 64) void k_hmean_partial(const Geo g, const State x, int f,
+                                                              const double* ttm, double* part,
+                                                              int npey, double cnt) {
+    constexpr int HM_SEG = hm_seg(NCH);
+    __shared__ __align__(16) double buf[2][NCH][HM_SEG + 2];
+    const int chains = (g.npz + 2) * npey, nry = g.npy / npey;
+    const int c0 = blockIdx.x * NCH, nc = min(NCH, chains - c0);
+    const long len = (long)g.npx * nry;
+    const int nseg = (int)((len + HM_SEG - 1) / HM_SEG);
+    // the summing wave: another one (another SIMD) in each round of blocks
+    const int wsum = (blockIdx.x >> 8) & 3, wave = threadIdx.x >> 6;
+    if (wave == wsum) {
+        const int c = threadIdx.x & 63;
+        double sum = 0.0;
+        for (int s = 0; s < nseg; ++s) {
+            __syncthreads();  // segment s is in LDS
+            if (c < nc) {
+                const double* v = buf[s & 1][c];
+                const int n = (int)min((long)HM_SEG, len - (long)s * HM_SEG);
+                int e = 0;
+                if (n == HM_SEG) {
+                    // four batches of 16 values in turn, each read three
+                    // batches (48 additions) before it is added; the
+                    // scheduling barriers keep that order
+                    constexpr int U = 8, NB = 4;
+                    double2 a[NB][U];
+                    auto rd = [&](double2* d, int at) {
 #pragma unroll
-            for (int u = 0; u < U2; ++u) v[u] = *(const double2*)(row + i + 2 * u);
+                        for (int u = 0; u < U; ++u) d[u] = *(const double2*)(v + at + 2 * u);
+                        __builtin_amdgcn_sched_barrier(0);
+                    };
 #pragma unroll
-            for (int u = 0; u < U2; ++u) {
-                sum += v[u].x;
-                sum += v[u].y;
+                    for (int b = 0; b < NB - 1; ++b) rd(a[b], 2 * U * b);
+#pragma unroll 1
+                    for (; e < HM_SEG; e += 2 * U * NB) {
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) {
+                            // (the last reads wrap round and are not used)
+                            rd(a[(b + NB - 1) % NB], (e + 2 * U * (b + NB - 1)) % HM_SEG);
+#pragma unroll
+                            for (int u = 0; u < U; ++u) {
+                                sum += a[b][u].x;
+                                sum += a[b][u].y;
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                } else {
+                    for (; e + 16 <= n; e += 16) {
+                        double a[16];
+#pragma unroll
+                        for (int u = 0; u < 16; ++u) a[u] = v[e + u];
+#pragma unroll
+                        for (int u = 0; u < 16; ++u) sum += a[u];
+                    }
+                    for (; e < n; ++e) sum += v[e];
+                }
             }
         }
-        for (; i + U <= g.npx; i += U) {
-            double v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = row[i + u];
-#pragma unroll
-            for (int u = 0; u < U; ++u) sum += v[u];
-        }
-        for (; i < g.npx; ++i) sum += row[i];
+        if (c < nc) part[c0 + c] = sum / cnt;
+        return;
     }
-    part[t] = sum / cnt;
-}
-__global__ __launch_bounds__(DEN_PARTIAL_THREADS) void k_den_partial(const Geo g,
-                                                                     const double* ro,
-                                                                     double* part, int npey,
-                                                                     double cnt) {
-    hmean_partial_chain(g, ro, part, npey, cnt);
-}
-
-// The convective flux WW2 = -RW*(2.5*(TT-TTM(K)) + 0.5*(UU*UU+VV*VV+WW*WW)),
-// UU = RU*(1/RO) (golden/fortran/3dmhdsub.f:1656-1666), of every interior
-// cell of planes 0..npz+1, into a field laid out like the state, so that
-// k_den_partial sums it with the reference's order.  One thread per cell:
-// the per-cell work (a division among it) runs at full occupancy instead of
-// inside the sequential sums.  grid = (row blocks, npy, npz + 2).
-__global__ __launch_bounds__(DEN_THREADS) void k_ww2_field(const Geo g, const State x,
-                                                           const double* ttm, double* w) {
-    const int i = 1 + blockIdx.x * DEN_THREADS + threadIdx.x, j = 1 + blockIdx.y, K = blockIdx.z;
-    if (i > g.npx) return;
-    const long n = g.at(i, j, K);
-    const double rw = x.q[QRW][n], ri = 1.0 / x.q[QRO][n];
-    const double uu = x.q[QRU][n] * ri, vv = x.q[QRV][n] * ri, ww = rw * ri;
-    w[n] = -rw * (2.5 * (x.q[QTT][n] - ttm[K]) + 0.5 * (uu * uu + vv * vv + ww * ww));
+    // A loading lane brings value t of each segment, for every chain of the
+    // block.  All its loads are unconditional, so that they are in flight
+    // together: past a chain's end it reads the chain's last row, past the
+    // last chain the last chain.
+    const int t = threadIdx.x - (wave > wsum ? 64 : 0);
+    constexpr int NV = WW2 ? 5 : 1;
+    double r[NCH][NV], tm[NCH];
+    int row = t / g.npx, col = t % g.npx;
+    const int drow = HM_SEG / g.npx, dcol = HM_SEG % g.npx;
+    long base[NCH];
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+        const int c = c0 + min(u, nc - 1);
+        base[u] = g.at(1, c % npey * nry + 1, c / npey);
+        tm[u] = WW2 ? ttm[c / npey] : 0.0;
+    }
+    auto fetch = [&] {  // the next segment; past the last it is not used
+        const long off = col + g.px * min(row, nry - 1);
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) {
+            if constexpr (WW2)
+                for (int q = 0; q < 5; ++q) r[u][q] = x.q[q][base[u] + off];
+            else
+                r[u][0] = x.q[f][base[u] + off];
+        }
+        row += drow;
+        col += dcol;
+        if (col >= g.npx) {
+            col -= g.npx;
+            row += 1;
+        }
+    };
+    fetch();
+    for (int s = 0; s < nseg; ++s) {
+        // buffer s & 1 was summed before the last barrier
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) {
+            const double* v = r[u];
+            double w = v[0];
+            if constexpr (WW2) {
+                const double rw = v[QRW], ri = 1.0 / v[QRO];
+                const double uu = v[QRU] * ri, vv = v[QRV] * ri, ww = rw * ri;
+                w = -rw * (2.5 * (v[QTT] - tm[u]) + 0.5 * (uu * uu + vv * vv + ww * ww));
+            }
+            buf[s & 1][u][t] = w;
+        }
+        fetch();
+        __syncthreads();
+    }
 }
 
 // The y ranks' partial means of one plane added in rank order.
@@ -226,20 +306,25 @@ __global__ __launch_bounds__(DEN_THREADS) void k_lrem_hrad(const double* ttm, do
               (ttm[K + 1] - ttm[K - 1]) * hz * dz * M.dkapa[K];
 }
 
-// Flux relaxation, one thread (golden/fortran/3dmhdsub.f:1625-1771, the
+// Flux relaxation, one block (golden/fortran/3dmhdsub.f:1625-1771, the
 // ITC=0 / IZC=1 branch): the TFAC update from the bottom-wall TTM, then per z
 // rank (nrz planes, the rank's lower ghost plane being the next rank's first)
 // FRADM, ALPHA and the trapezoid integral CORRECT, offset by the sum of the
 // ranks above's end values, and ftc = RLAX*TFAC*CORRECT for the interior.
-// One block.  ALPHA depends on the plane only (a rank's lower ghost plane
-// takes the next rank's FRADM, which is that plane's own centred value), so
-// the block computes it for planes 1..npz+1 first; thread 0 then runs the
-// chain, reading ALPHA and ZEE eight planes ahead of the in-order sums.
+// ALPHA depends on the plane only (a rank's lower ghost plane takes the next
+// rank's FRADM, which is that plane's own centred value), and so does a
+// trapezoid 0.5*(ALPHA(k)+ALPHA(k-1))*(ZEE(k)-ZEE(k-1)): the block forms both
+// for every plane, in parallel.  Only the sums run in order: one lane per rank
+// adds its nrz trapezoids (a rank's CORRECT starts from zero), one lane the
+// ranks' end values, and the block forms ftc.  One lane doing all of it took
+// 54 us a stage at npz 512, this takes 14.
 constexpr int RLX_THREADS = 256;
 __global__ __launch_bounds__(RLX_THREADS) void k_rlax_chain(
     const DevScal* sc, int stage, double* st, const double* ttm, const double* fconm, double* alpha,
     double* ftc, const Metrics M, int npz, int npez, double hz, double repr, double theta,
-    double rlax, double tstart, double toff) {
+    double rlax, double tstart, double toff, double* offset) {
+    __shared__ double rt_s;
+    __shared__ int on_s;
     const double ftot = theta / repr;
     for (int G = 1 + threadIdx.x; G <= npz + 1; G += RLX_THREADS) {
         double fr;
@@ -256,60 +341,76 @@ __global__ __launch_bounds__(RLX_THREADS) void k_rlax_chain(
         double a = 1.0 - (fconm[G] + fr) / ftot;
         alpha[G] = a / (1.0 + 4.0 * fabs(a));
     }
+    if (threadIdx.x == 0) {
+        const double dt = stage == 0 ? sc->dt_next : sc->dt;  // the step's dt
+        const double timt = sc->timc + sc->timi;
+        double tfac = st[0];
+        const bool on = timt > tstart && tfac > 1e-4;
+        if (on) {
+            const double tbot = ttm[npz];
+            if (tbot <= st[1]) {
+                tfac = tfac - dt / (3.0 * toff);
+            } else {
+                st[1] = tbot;
+                tfac = tfac + dt / (3.0 * toff);
+                tfac = fmin(tfac, 2.0);
+            }
+            st[0] = tfac;
+        }
+        rt_s = rlax * tfac;
+        on_s = on;
+    }
     __threadfence_block();
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    const double dt = stage == 0 ? sc->dt_next : sc->dt;  // the step's dt
-    const double timt = sc->timc + sc->timi;
-    double tfac = st[0];
-    const bool on = timt > tstart && tfac > 1e-4;
-    if (on) {
-        const double tbot = ttm[npz];
-        if (tbot <= st[1]) {
-            tfac = tfac - dt / (3.0 * toff);
-        } else {
-            st[1] = tbot;
-            tfac = tfac + dt / (3.0 * toff);
-            tfac = fmin(tfac, 2.0);
-        }
-        st[0] = tfac;
-    }
-    const double rt = rlax * tfac;
-    if (!on) {
-        for (int G = 1; G <= npz; ++G) ftc[G] = rt * 0.0;
+    const double rt = rt_s;
+    if (!on_s) {
+        for (int G = 1 + threadIdx.x; G <= npz; G += RLX_THREADS) ftc[G] = rt * 0.0;
         return;
     }
+    // the trapezoid that ends at plane G (2..npz+1), into ftc[G]
+    for (int G = 2 + threadIdx.x; G <= npz + 1; G += RLX_THREADS)
+        ftc[G] = 0.5 * (alpha[G] + alpha[G - 1]) * (M.zee[G] - M.zee[G - 1]);
+    __threadfence_block();
+    __syncthreads();
+    // CORRECT(k) = CORRECT(k-1) + trapezoid(k), k = 2..nrz+1 of the rank
+    // (global G0+k), into alpha; CORRECT(nrz+1) is the rank's end value
     const int nrz = npz / npez;
-    double sum = 0.0;  // end values of the ranks above, added in rank order
-    for (int pz = 0; pz < npez; ++pz) {
+    for (int pz = threadIdx.x; pz < npez; pz += RLX_THREADS) {
         const int G0 = pz * nrz;
         double corr = 0.0;
-        // CORRECT(k) = CORRECT(k-1) + 0.5*(ALPHA(k)+ALPHA(k-1))*(ZEE(k)-ZEE(k-1)),
-        // k = 2..nrz+1 of the rank (global G0+k)
+        alpha[G0 + 1] = corr;
+        constexpr int U = 16;
         int k = 2;
-        constexpr int U = 8;
-        for (; k + U - 1 <= nrz + 1; k += U) {
-            double ap[U + 1], zp[U + 1];
+        for (; k + U - 1 <= nrz; k += U) {
+            double t[U];
 #pragma unroll
-            for (int u = 0; u <= U; ++u) {
-                ap[u] = alpha[G0 + k - 1 + u];
-                zp[u] = M.zee[G0 + k - 1 + u];
-            }
-            if (k == 2) ftc[G0 + 1] = rt * (corr + sum);
+            for (int u = 0; u < U; ++u) t[u] = ftc[G0 + k + u];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                corr = corr + 0.5 * (ap[u + 1] + ap[u]) * (zp[u + 1] - zp[u]);
-                if (k + u <= nrz) ftc[G0 + k + u] = rt * (corr + sum);
+                corr = corr + t[u];
+                alpha[G0 + k + u] = corr;
             }
         }
-        if (k == 2) ftc[G0 + 1] = rt * (corr + sum);
-        for (; k <= nrz + 1; ++k) {
-            const int G = G0 + k;
-            corr = corr + 0.5 * (alpha[G] + alpha[G - 1]) * (M.zee[G] - M.zee[G - 1]);
-            if (k <= nrz) ftc[G] = rt * (corr + sum);
+        for (; k <= nrz; ++k) {
+            corr = corr + ftc[G0 + k];
+            alpha[G0 + k] = corr;
         }
-        sum = sum + corr;  // this rank's end value, CORRECT(NZ)
+        offset[pz] = corr + ftc[G0 + nrz + 1];
     }
+    __threadfence_block();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double sum = 0.0;  // end values of the ranks above, added in rank order
+        for (int pz = 0; pz < npez; ++pz) {
+            const double end = offset[pz];
+            offset[pz] = sum;
+            sum = sum + end;
+        }
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int G = 1 + threadIdx.x; G <= npz; G += RLX_THREADS)
+        ftc[G] = rt * (alpha[G] + offset[(G - 1) / nrz]);
 }
 
 
@@ -518,6 +619,30 @@ void launch_stage_kernel(r3d_hip_ctx* c, const StageArgs& a, int stage, int zmod
 #undef R3D_STAGE
 }
 
+// Per-(plane, y rank) partial means of field f of the current state into
+// den_buf, or (ttm given) those of the convective flux.
+void launch_hmean_partial(r3d_hip_ctx* c, int f, const double* ttm) {
+    const r3d_hip_cfg& p = c->cfg;
+    State s;
+    for (int q = 0; q < NXF; ++q) s.q[q] = c->xs[c->cur][q];
+    const int chains = (p.npz + 2) * p.npey;
+    const double cnt = (double)(p.npx * p.npy);
+#define R3D_HM(N, W)                                                                         \
+    hipLaunchKernelGGL((k_hmean_partial<N, W>), dim3((chains + N - 1) / N), dim3(hm_seg(N) + 64), \
+                       0, c->stream, c->g, s, f, ttm, c->den_buf, p.npey, cnt)
+    if (chains <= c->cus) {
+        if (ttm) R3D_HM(1, true);
+        else R3D_HM(1, false);
+    } else if (ttm) {
+        R3D_HM(4, true);
+    } else if (chains <= 4 * c->cus) {
+        R3D_HM(4, false);
+    } else {
+        R3D_HM(8, false);
+    }
+#undef R3D_HM
+}
+
 // Density diffusion set-up of this stage's input: mirrored outer RO planes,
 // horizontal mean ROM and the per-plane coefficients.
 int launch_density_prep(r3d_hip_ctx* c) {
@@ -526,10 +651,7 @@ int launch_density_prep(r3d_hip_ctx* c) {
     const int nk = f.npz + 2, cells = (f.npx + 2) * (f.npy + 2);
     hipLaunchKernelGGL(k_den_mirror, dim3((cells + DEN_THREADS - 1) / DEN_THREADS),
                        dim3(DEN_THREADS), 0, c->stream, c->g, ro);
-    hipLaunchKernelGGL(k_den_partial,
-                       dim3((nk * f.npey + DEN_PARTIAL_THREADS - 1) / DEN_PARTIAL_THREADS),
-                       dim3(DEN_PARTIAL_THREADS), 0, c->stream, c->g, (const double*)ro, c->den_buf,
-                       f.npey, (double)(f.npx * f.npy));
+    launch_hmean_partial(c, QRO, nullptr);
     const size_t nkz = (size_t)nk;
     double* rom = c->den_buf + nkz * f.npey;
     hipLaunchKernelGGL(k_den_final, dim3((nk + DEN_THREADS - 1) / DEN_THREADS), dim3(DEN_THREADS),
@@ -553,25 +675,17 @@ int launch_relax_prep(r3d_hip_ctx* c, int stage) {
     double* ftc = fconm + nkz;
     double* alpha = ftc + nkz;
     double* st = c->den_buf + nkz * (f.npey + 9);
-    State s;
-    for (int q = 0; q < NXF; ++q) s.q[q] = c->xs[c->cur][q];
-    const double cnt = (double)(f.npx * f.npy);
-    const dim3 gp((nk * f.npey + DEN_PARTIAL_THREADS - 1) / DEN_PARTIAL_THREADS);
     const dim3 gf((nk + DEN_THREADS - 1) / DEN_THREADS);
-    hipLaunchKernelGGL(k_den_partial, gp, dim3(DEN_PARTIAL_THREADS), 0, c->stream, c->g,
-                       (const double*)s.q[QTT], part, f.npey, cnt);
+    launch_hmean_partial(c, QTT, nullptr);
     hipLaunchKernelGGL(k_hmean_final, gf, dim3(DEN_THREADS), 0, c->stream, (const double*)part, ttm,
                        nk, f.npey);
-    hipLaunchKernelGGL(k_ww2_field, dim3((f.npx + DEN_THREADS - 1) / DEN_THREADS, f.npy, nk),
-                       dim3(DEN_THREADS), 0, c->stream, c->g, s, (const double*)ttm, c->ww2_buf);
-    hipLaunchKernelGGL(k_den_partial, gp, dim3(DEN_PARTIAL_THREADS), 0, c->stream, c->g,
-                       (const double*)c->ww2_buf, part, f.npey, cnt);
+    launch_hmean_partial(c, QTT, ttm);
     hipLaunchKernelGGL(k_hmean_final, gf, dim3(DEN_THREADS), 0, c->stream, (const double*)part,
                        fconm, nk, f.npey);
     hipLaunchKernelGGL(k_rlax_chain, dim3(1), dim3(RLX_THREADS), 0, c->stream,
                        (const DevScal*)c->scal, stage, st, (const double*)ttm, (const double*)fconm,
                        alpha, ftc, c->M, f.npz, f.npez, f.hz, f.repr, f.theta, f.rlax, f.tstart,
-                       f.toff);
+                       f.toff, st + 2);
     HIPCHK(hipGetLastError());
     return R3D_OK;
 }
@@ -585,11 +699,8 @@ int launch_lrem_prep(r3d_hip_ctx* c) {
     double* part = c->den_buf;
     double* ttm = c->den_buf + nkz * (f.npey + 4);
     double* hrad = c->den_buf + nkz * (f.npey + 8);
-    const dim3 gp((nk * f.npey + DEN_PARTIAL_THREADS - 1) / DEN_PARTIAL_THREADS);
     const dim3 gf((nk + DEN_THREADS - 1) / DEN_THREADS);
-    hipLaunchKernelGGL(k_den_partial, gp, dim3(DEN_PARTIAL_THREADS), 0, c->stream, c->g,
-                       (const double*)c->xs[c->cur][QTT], part, f.npey,
-                       (double)(f.npx * f.npy));
+    launch_hmean_partial(c, QTT, nullptr);
     hipLaunchKernelGGL(k_hmean_final, gf, dim3(DEN_THREADS), 0, c->stream, (const double*)part, ttm,
                        nk, f.npey);
     hipLaunchKernelGGL(k_lrem_hrad, gf, dim3(DEN_THREADS), 0, c->stream, (const double*)ttm, hrad,
@@ -820,6 +931,7 @@ int r3d_hip_create(const r3d_hip_cfg* cfg, r3d_hip_ctx** out) {
 
     auto* c = new r3d_hip_ctx();
     c->cfg = f;
+    c->cus = cus;
     c->nf = f.lmag ? 8 : 5;
     c->g.npx = f.npx;
     c->g.npy = f.npy;
@@ -900,14 +1012,16 @@ int r3d_hip_create(const r3d_hip_cfg* cfg, r3d_hip_ctx** out) {
     if ((rc = dev_alloc(c, &c->metric_buf, nmet))) return fail(rc);
     if (f.id != 0 || f.rlax > 0.0 || f.lrem) {
         // rows of npz+2: npey partial means, ROM, DH*ORE*WWZ, DV*ORE*WWZ, the ID=2
-        // profile, TTM, FCONM, RLAX*TFAC*CORRECT, ALPHA, HRAD; then TFAC, TTM_MAX
-        const size_t nk = (size_t)f.npz + 2, n = nk * ((size_t)f.npey + 9) + 2;
+        // profile, TTM, FCONM, RLAX*TFAC*CORRECT, ALPHA, HRAD; then TFAC, TTM_MAX and
+        // npez rank offsets of CORRECT
+        const size_t nk = (size_t)f.npz + 2, rows = nk * ((size_t)f.npey + 9);
+        const size_t n = rows + 2 + f.npez;
         if ((rc = dev_alloc(c, &c->den_buf, n))) return fail(rc);
         // zero rows the run does not compute; TFAC = 1, TTM_MAX = -1e99
         // (DATA statements, golden/fortran/3dmhdsub.f:1258-1259)
         std::vector<double> init(n, 0.0);
-        init[n - 2] = 1.0;
-        init[n - 1] = -1e99;
+        init[rows] = 1.0;
+        init[rows + 1] = -1e99;
         if (hipMemcpy(c->den_buf, init.data(), n * sizeof(double), hipMemcpyHostToDevice) !=
             hipSuccess)
             return fail(set_err(R3D_EHIP, "hipMemcpy of the per-plane buffer failed"));
@@ -918,7 +1032,6 @@ int r3d_hip_create(const r3d_hip_cfg* cfg, r3d_hip_ctx** out) {
         c->M.ttm = c->M.rom + 4 * nk;
         c->M.hrad = c->M.rom + 8 * nk;
     }
-    if (f.rlax > 0.0 && (rc = dev_alloc(c, &c->ww2_buf, field_elems(c->g)))) return fail(rc);
     const size_t stage_elems = (size_t)std::max<long>((long)c->nx * c->ny * c->nz,
                                                       (long)(f.npx + 2) * (f.npy + 2));
     if ((rc = dev_alloc(c, &c->stage_buf, stage_elems))) return fail(rc);
@@ -942,7 +1055,6 @@ int r3d_hip_destroy(r3d_hip_ctx* c) {
     if (c->scal) (void)hipFree(c->scal);
     if (c->metric_buf) (void)hipFree(c->metric_buf);
     if (c->den_buf) (void)hipFree(c->den_buf);
-    if (c->ww2_buf) (void)hipFree(c->ww2_buf);
     if (c->stage_buf) (void)hipFree(c->stage_buf);
     if (c->gstage) (void)hipFree(c->gstage);
     if (c->copy_stream) {
