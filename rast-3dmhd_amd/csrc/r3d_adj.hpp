@@ -750,13 +750,13 @@ struct MagWallAdj {
     double rw2, ro2, bx2, by2, bx3, by3;
 };
 
-// cell_flux_mag_extra_vjp in point-major form, for kernels that add each
-// adjoint entry into an accumulator as soon as it is known: the cell's
+// cell_flux_mag_extra_vjp in point-major form, a second statement of the same
+// transpose that the CPU check holds the first against: the cell's
 // coefficients (adjoints of the derivatives of B and of the velocities,
 // the resistive Laplacian weights) first, then each face point's seven
 // entries in closed form, so that no per-point adjoint array is held.
 // pt(q, ri, u, v, w) returns 1/RO and the velocities at face point q (a
-// kernel re-reads them where they are needed); out(q, f, value) receives the
+// caller re-reads them where they are needed); out(q, f, value) receives the
 // entry of primary f (QRU..QRO, QBX..QBZ; the temperature's is zero) at face
 // point q, each (q, f) once.  The same entries as cell_flux_mag_extra_vjp,
 // which sums some of them in another order.
