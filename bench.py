@@ -507,12 +507,10 @@ def measure_steps(pkg, args, variant, steps, warmup):
     sim.sync()
     wall = time.perf_counter() - t0
     n_stage, ms_stage = sim.kernel_stats(0)
-    n_bound, ms_bound = sim.kernel_stats(1)
     sim.set_timing(False)
     sc = sim.scalars()
     log(f"[bench] nit={sc['nit']} dt={sc['dt']:.6g} umach={sc['umach']:.6g}; "
-        f"stage kernel {n_stage} launches avg {ms_stage / max(n_stage, 1):.3f} ms, "
-        f"boundary kernel avg {ms_bound / max(n_bound, 1):.3f} ms")
+        f"stage kernel {n_stage} launches avg {ms_stage / max(n_stage, 1):.3f} ms")
     sim.close()
     return wall, ms_stage / max(n_stage, 1) / 1e3, mem
 

@@ -526,7 +526,7 @@ int get_state(r3d_adj_ctx* a, double* dst) {
 }
 
 // The stage kernels write interior cells only, and the outer z planes keep
-// X0's values (RO's is rewritten by the boundary kernel every stage), so a
+// X0's values (RO's is rewritten by every stage), so a
 // buffer that a stage writes into must hold them: copy X0's planes 0 and
 // npz+1 into every segment buffer, once per initial state.
 // The final state of the forward is the last stage's output buffer: it gets

@@ -1,13 +1,5 @@
-// r3d_aux.hpp - boundary-plane, dt and bookkeeping kernels (gfx950).
+// r3d_aux.hpp - halo, dt and bookkeeping kernels (gfx950).
 //
-// k_bound   : per stage, after k_stage.  BCON on the global top (k = 1) and
-//             bottom (k = npz) planes (reference src/bcon.cpp:12-141, with
-//             BZ = 0 under LMAG), the
-//             deferred Z' mix on those planes, their dt limits in the last
-//             stage, and the
-//             1/RO flip of the two outer ghost planes that the reference's
-//             FLUXES performs on its full array (src/fluxes.cpp:133-138) but
-//             its halo exchange never refreshes.
 // halo_thread: periodic x/y ghost images of a state, written before a download
 //             (the step itself reads wrapped interior cells instead).
 // k_dt      : dt limits of the current state when no fused value is
@@ -19,110 +11,7 @@
 
 namespace R3D_KNS {
 
-constexpr int BOUND_THREADS = 256;
 constexpr int DT_THREADS = 256;
-
-// Block bx of nbb (per side) of the boundary pass, NT threads a block; side
-// 0 = top, 1 = bottom.  Its dt partial goes to slot partial_base + side * nbb
-// + bx.
-template <int NT = BOUND_THREADS>
-__device__ __forceinline__ void bound_block(const StageArgs& a, const Consts& C, const Metrics& M,
-                                            int partial_base, int bx, int nbb, int side) {
-    __shared__ double red[NT / 64][NPART];
-    const Geo g = a.g;
-    const int W = g.npx + 2, H = g.npy + 2;
-    const int idx = bx * NT + threadIdx.x;
-    double pm[NPART] = {0.0, 1e300, 1e300, 1e300, 1e300};
-    const double dt = a.scal->dt;
-    const double cz = (a.stage < 2) ? C.zeta[a.stage] * dt : 0.0;
-
-    if (idx < W * H) {
-        const int i = idx % W, j = idx / W;
-        // outer ghost plane: RO <- 1/RO over the whole plane
-        const long no = g.at(i, j, side ? g.npz + 1 : 0);
-        a.xout.q[QRO][no] = 1.0 / a.xin.q[QRO][no];
-
-        if (i >= 1 && i <= g.npx && j >= 1 && j <= g.npy) {
-            const int kb = side ? g.npz : 1;
-            const long n = g.at(i, j, kb);
-            const long d1 = side ? -g.pp : g.pp;
-            double* const* X = a.xout.q;
-            const double ro = X[QRO][n], ro1 = X[QRO][n + d1], ro2 = X[QRO][n + 2 * d1];
-            const double ru = ro * (C.c43 * X[QRU][n + d1] / ro1 - C.c13 * X[QRU][n + 2 * d1] / ro2);
-            const double rv = ro * (C.c43 * X[QRV][n + d1] / ro1 - C.c13 * X[QRV][n + 2 * d1] / ro2);
-            const double rw = 0.0;
-            double tt = X[QTT][n];
-            const double tt1 = X[QTT][n + d1], tt2 = X[QTT][n + 2 * d1];
-            if (side == 0) {
-                switch (C.top_mode) {
-                    case TOP_GAUSS_T:
-                        tt = 1.0 - (1.0 - C.tpr) * M.e1[i] / C.hh * M.e2[j] / C.hh;
-                        break;
-                    case TOP_GAUSS_FLUX:
-                        tt = C.c43 * tt1 - C.c13 * tt2 -
-                             C.c23 * M.dz_top *
-                                 (C.theta - (C.theta - C.tpr) * M.e1[i] / C.hh * M.e2[j] / C.hh);
-                        break;
-                    case TOP_CONST_T:  // LREM: TU (golden/fortran/3dmhdsub.f:2852-2853)
-                        tt = C.lrem ? C.tu : 1.0;
-                        if (!C.lrem && C.half_t && i <= (g.npx + 2) / 2) tt = 1.0 - C.tp;
-                        break;
-                    case TOP_CONST_FLUX:  // LREM: + DZTU (:2876-2879)
-                        tt = C.lrem ? C.c43 * tt1 - C.c13 * tt2 + C.dztu
-                                    : C.c43 * tt1 - C.c13 * tt2 - C.c23 * M.dz_top * C.theta;
-                        break;
-                    default:
-                        break;
-                }
-            } else {
-                if (C.izcon == 0)
-                    tt = C.tb;
-                else if (C.lrem)  // + DZTB (golden/fortran/3dmhdsub.f:2949-2952)
-                    tt = C.c43 * tt1 - C.c13 * tt2 + C.dztb;
-                else
-                    tt = C.c43 * tt1 - C.c13 * tt2 + C.c23 * M.dz_bot * C.theta / M.rkapa[kb];
-            }
-            X[QRU][n] = ru;
-            X[QRV][n] = rv;
-            X[QRW][n] = rw;
-            X[QTT][n] = tt;
-            // LMAG: BZ = 0 on both walls (src/bcon.cpp:95-98, 136-139); BX, BY
-            // keep their updated values
-            double bx = 0.0, by = 0.0, bz = 0.0;
-            if (C.lmag) {
-                bx = X[QBX][n];
-                by = X[QBY][n];
-                bz = C.bz_zero ? 0.0 : X[QBZ][n];
-                X[QBZ][n] = bz;
-            }
-
-            if (a.zmode == 0 && a.stage < 2) {
-                // mix for the next stage with the post-BCON state; the stage
-                // kernel left F in Z on this plane
-                double* const* Z = a.z.q;
-                Z[QRU][n] = ru + cz * Z[QRU][n];
-                Z[QRV][n] = rv + cz * Z[QRV][n];
-                Z[QRW][n] = rw + cz * Z[QRW][n];
-                Z[QRO][n] = ro + cz * Z[QRO][n];
-                Z[QTT][n] = tt + cz * Z[QTT][n];
-                if (C.lmag) {
-                    Z[QBX][n] = bx + cz * Z[QBX][n];
-                    Z[QBY][n] = by + cz * Z[QBY][n];
-                    Z[QBZ][n] = bz + cz * Z[QBZ][n];
-                }
-            }
-            if (a.stage == 2 && a.want_dt) {
-                const double dd = dmin(dmin(M.ddx[i], M.ddy[j]), M.ddz[kb]);
-                if (C.lmag)
-                    dt_terms<true>(C, ru, rv, rw, ro, tt, bx, by, bz, dd, M.rkdt[kb], pm);
-                else
-                    dt_terms<false>(C, ru, rv, rw, ro, tt, 0.0, 0.0, 0.0, dd, M.rkdt[kb], pm);
-            }
-        }
-    }
-    if (a.stage == 2 && a.want_dt)
-        block_partials<NT / 64>(pm, red, a.partial, partial_base + side * nbb + bx);
-}
 
 // dt limits of the state `s` (reference src/step.cpp:121-209): block bx of
 // nbx (NT threads each), one partial per block.
@@ -230,5 +119,27 @@ __device__ __forceinline__ void finish_block(DevScal* sc, const double* partial,
     }
 }
 
+// The exact dt pass after a screened reduction that could not prove its
+// extrema (DevScal::dt_redo): block bx of nbx reduces its share of the state,
+// and the block that ends last reduces the partials (both in one launch, which
+// costs a step 2 us when there is nothing to do).  Every thread reads the
+// flag at its block's start; the last block clears it, when all have started.
+template <int NT = DT_THREADS>
+__device__ __forceinline__ void redo_block(const Geo& g, const State& s, const Consts& C,
+                                           const Metrics& M, double* partial, DevScal* sc, int bx,
+                                           int nbx) {
+    if (!sc->dt_redo) return;
+    __shared__ int last;
+    dt_block<NT>(g, s, C, M, partial, bx, nbx);
+    if (threadIdx.x == 0) {
+        __threadfence();  // this block's partial, written by this thread
+        last = atomicAdd(&sc->redo_done, 1) == nbx - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();  // the other blocks' partials
+    finish_block<NT>(sc, partial, nbx, C, 1, 0, 0);
+    if (threadIdx.x == 0) sc->redo_done = 0;
+}
 
 }  // namespace R3D_KNS

@@ -64,7 +64,7 @@ struct r3d_hip_ctx {
     bool metrics_set = false;
     bool next_valid = false;  // scal->dt_next holds the dt of the current state
     std::vector<char> uploaded;
-    int ty = r3d::TILE_Y, tw = 64, ntx = 0, nty = 0, nkc = 0, kc = 0, kq = 0, krem = 0, nblocks = 0, grid = 0, nbb = 0;
+    int ty = r3d::TILE_Y, tw = 64, ntx = 0, nty = 0, nkc = 0, kc = 0, kq = 0, krem = 0, nblocks = 0, grid = 0;
     unsigned long long bytes = 0;
     bool timing = false;
     long launches[4] = {0, 0, 0, 0};

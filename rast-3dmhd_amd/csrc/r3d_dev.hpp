@@ -39,8 +39,8 @@ struct DevScal {
     // the last reduction's extrema: the least time-step limit over all cells
     // and limits, and the largest ogamma*UU/T; they set the next screen (below)
     double lim_prev, um_prev;
-    int dt_redo;  // the screened reduction could not prove its extrema: redo exactly
-    int pad2;
+    int dt_redo;    // the screened reduction could not prove its extrema: redo exactly
+    int redo_done;  // blocks of that exact pass that have written their partial
 };
 
 // Time-step screen of stage 3.  A cell's limits can only set the next dt if

@@ -5,8 +5,8 @@
 // descriptor per member and launches each RK stage once for all members: the
 // global tile index of a block is mapped to (member, tile) through the
 // members' first-tile offsets, so a stage of 64 small runs fills the GPU the
-// way one large run does.  The boundary pass, the dt reductions and the
-// end-of-step bookkeeping are likewise one launch each, indexed by member.
+// way one large run does.  The dt reductions and the end-of-step bookkeeping
+// are likewise one launch each, indexed by member.
 // A step is captured in a HIP graph per X parity and replayed.
 #include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
@@ -29,8 +29,7 @@ struct EnsMember {
     State z;
     double* partial;
     DevScal* scal;
-    int ntx, nty, nkc, kc, nblocks, nbb, tile0, npart_dt;
-    int bnd0, nbbp;  // persistent launch: first boundary unit, boundary blocks per side
+    int ntx, nty, nkc, kq, krem, nblocks, tile0, npart_dt;
     Consts C;
     Metrics M;
 };
@@ -53,10 +52,32 @@ __device__ __forceinline__ StageArgs member_args(const EnsMember& e, int cur, in
     a.ntx = e.ntx;
     a.nty = e.nty;
     a.nkc = e.nkc;
-    a.kq = e.kc;
-    a.krem = 0;
+    a.kq = e.kq;
+    a.krem = e.krem;
     a.nblocks = e.nblocks;
     return a;
+}
+
+// One tile of one stage of member e, then its wall cells (member data read by a
+// second route there, as in k_stage), then its dt partial.
+template <int TY, int STAGE, bool MAG, int TW>
+__device__ __forceinline__ void member_tile(const EnsMember& e, int t, int cur,
+                                            StageLds<TY, STAGE, MAG, false, false, TW>& lds) {
+    constexpr int ZMODE = STAGE < 2 ? 0 : 2;
+    double pm[NPART];
+    TileCell<TY, TW> me;
+    // copies: read through the table the constants would be loaded again after
+    // every store of the z loop, which might alias it
+    const StageArgs a = member_args(e, cur, STAGE, ZMODE, STAGE == 2);
+    const Consts C = e.C;
+    const Metrics M = e.M;
+    if (stage_tile<TY, STAGE, ZMODE, MAG, false, false, TW>(a, C, M, t, lds, pm, me)) {
+        const EnsMember* w = &e;
+        asm volatile("" : "+s"(w));
+        stage_walls<TY, STAGE, ZMODE, MAG, TW>(member_args(*w, cur, STAGE, ZMODE, STAGE == 2),
+                                               w->C, w->M, me, pm);
+    }
+    if (STAGE == 2) block_partials<TileShape<TY, TW>::NW>(pm, lds.red, a.partial, t);
 }
 
 // One stage of a full step for every member.  Tiles of one member are
@@ -75,9 +96,7 @@ __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_stage_ens(
         else hi = mid - 1;
     }
     const EnsMember& e = mem[lo];
-    constexpr int ZMODE = STAGE < 2 ? 0 : 2;
-    const StageArgs a = member_args(e, cur, STAGE, ZMODE, STAGE == 2);
-    stage_tile<TY, STAGE, ZMODE, MAG, false, false, TW>(a, e.C, e.M, T - e.tile0, lds);
+    member_tile<TY, STAGE, MAG, TW>(e, T - e.tile0, cur, lds);
 }
 
 // Last member m with key(mem[m]) <= v (keys ascending from mem[0] = 0).
@@ -97,7 +116,7 @@ __device__ __forceinline__ int find_member(const EnsMember* mem, int nmem, int v
 // size).  Each phase is a loop of its blocks over work units, followed by a
 // grid-wide barrier (cooperative groups: every block writes its L2 back and
 // invalidates it, so a phase sees the previous phase's stores on every XCD):
-//   per stage: the stage tiles, then the boundary pass;
+//   per stage: the stage tiles;
 //   per step: each member's dt reduction with the screen's proof, then, only
 //   when some member's proof failed, the exact pass and its reduction for
 //   those members.
@@ -115,8 +134,7 @@ __device__ __forceinline__ int find_member(const EnsMember* mem, int nmem, int v
 // how the partials are grouped).  work[0..8] must be zero at launch.
 template <int TY, bool MAG, int TW>
 __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_ens_run(
-    const EnsMember* __restrict__ mem, int nmem, int ntiles, int nbunits, int cur, int nsteps,
-    int* work) {
+    const EnsMember* __restrict__ mem, int nmem, int ntiles, int cur, int nsteps, int* work) {
     constexpr int NT = TileShape<TY, TW>::NW * 64;
     __shared__ union {
         StageLds<TY, 0, MAG, false, false, TW> s0;
@@ -137,37 +155,27 @@ __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_ens_run(
             for (;;) {
                 if (threadIdx.x == 0) grab = atomicAdd(&work[xcd], 1) - base;
                 __syncthreads();
-                const int i = grab;
+                const int i = __builtin_amdgcn_readfirstlane(grab);
                 __syncthreads();  // grab is rewritten by the next take
                 if (i >= n_x) break;
                 const int T = xcd * tiles_xcd + i;
                 const EnsMember& e =
                     mem[find_member(mem, nmem, T, [](const EnsMember& x) { return x.tile0; })];
-                const StageArgs a = member_args(e, cur, s, s < 2 ? 0 : 2, s == 2);
                 if (s == 0)
-                    stage_tile<TY, 0, 0, MAG, false, false, TW>(a, e.C, e.M, T - e.tile0, lds.s0);
+                    member_tile<TY, 0, MAG, TW>(e, T - e.tile0, cur, lds.s0);
                 else if (s == 1)
-                    stage_tile<TY, 1, 0, MAG, false, false, TW>(a, e.C, e.M, T - e.tile0, lds.s1);
+                    member_tile<TY, 1, MAG, TW>(e, T - e.tile0, cur, lds.s1);
                 else
-                    stage_tile<TY, 2, 2, MAG, false, false, TW>(a, e.C, e.M, T - e.tile0, lds.s2);
+                    member_tile<TY, 2, MAG, TW>(e, T - e.tile0, cur, lds.s2);
                 __syncthreads();  // the next tile reuses the LDS
             }
             base += n_x + per_xcd;
-            grid.sync();
-            for (int u = blockIdx.x; u < nbunits; u += nblk) {
-                const EnsMember& e =
-                    mem[find_member(mem, nmem, u, [](const EnsMember& x) { return x.bnd0; })];
-                const int l = u - e.bnd0;
-                const StageArgs a = member_args(e, cur, s, s < 2 ? 0 : 2, s == 2);
-                bound_block<NT>(a, e.C, e.M, e.nblocks, l % e.nbbp, e.nbbp, l / e.nbbp);
-                __syncthreads();
-            }
             grid.sync();
             cur ^= 1;
         }
         for (int m = blockIdx.x; m < nmem; m += nblk) {
             const EnsMember& e = mem[m];
-            finish_block<NT>(e.scal, e.partial, e.nblocks + 2 * e.nbbp, e.C, 1, 1, 1);
+            finish_block<NT>(e.scal, e.partial, e.nblocks, e.C, 1, 1, 1);
             if (threadIdx.x == 0 && e.scal->dt_redo) work[8] = 1;
             __syncthreads();
         }
@@ -196,15 +204,6 @@ __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_ens_run(
     }
 }
 
-// grid = (max boundary blocks, 2 sides, members)
-__global__ __launch_bounds__(BOUND_THREADS) void k_bound_ens(const EnsMember* __restrict__ mem,
-                                                             int cur, int stage) {
-    const EnsMember& e = mem[blockIdx.z];
-    if ((int)blockIdx.x >= e.nbb) return;
-    const StageArgs a = member_args(e, cur, stage, stage < 2 ? 0 : 2, stage == 2);
-    bound_block(a, e.C, e.M, e.nblocks, blockIdx.x, e.nbb, blockIdx.y);
-}
-
 // grid = (ENS_DT_BLOCKS, members)
 __global__ __launch_bounds__(DT_THREADS) void k_dt_ens(const EnsMember* __restrict__ mem,
                                                        int cur) {
@@ -217,25 +216,16 @@ __global__ __launch_bounds__(DT_THREADS) void k_dt_ens(const EnsMember* __restri
 __global__ __launch_bounds__(1024) void k_finish_ens(const EnsMember* __restrict__ mem,
                                                      int fused, int advance) {
     const EnsMember& e = mem[blockIdx.x];
-    finish_block(e.scal, e.partial, fused ? e.nblocks + 2 * e.nbb : e.npart_dt, e.C, 1, advance,
+    finish_block(e.scal, e.partial, fused ? e.nblocks : e.npart_dt, e.C, 1, advance,
                  fused);
 }
 
-// The exact dt pass of the members whose screened extrema were not proven
-// (DevScal::dt_redo); the blocks of every other member return at once.
+// The exact dt pass of the members whose screened extrema were not proven.
 // grid = (ENS_DT_BLOCKS, members)
 __global__ __launch_bounds__(DT_THREADS) void k_dt_redo_ens(const EnsMember* __restrict__ mem,
                                                             int cur) {
     const EnsMember& e = mem[blockIdx.y];
-    if (!e.scal->dt_redo) return;
-    dt_block(e.g, e.x[cur], e.C, e.M, e.partial, blockIdx.x, gridDim.x);
-}
-// grid = (members): all threads read the flag before the reduction's first
-// barrier; thread 0 clears it after the last
-__global__ __launch_bounds__(1024) void k_finish_redo_ens(const EnsMember* __restrict__ mem) {
-    const EnsMember& e = mem[blockIdx.x];
-    if (!e.scal->dt_redo) return;
-    finish_block(e.scal, e.partial, e.npart_dt, e.C, 1, 0, 0);
+    redo_block(e.g, e.x[cur], e.C, e.M, e.partial, e.scal, blockIdx.x, gridDim.x);
 }
 
 // Stage tiles of the ensemble: ty rows, kc planes (0: 32), tw columns (64,
@@ -256,17 +246,17 @@ struct r3d_ens_ctx {
     hipStream_t stream = nullptr;
     int device = 0, lmag = 0;
     Tiling tile{8, 0, 64};
-    int ntiles = 0, grid = 0, nbb_max = 0;
+    int ntiles = 0, grid = 0;
     int cur = 0;
     bool use_graph = true;
     bool persistent = false;  // one cooperative launch per r3d_ens_step call
-    int nbunits = 0;          // persistent launch: boundary units of all members
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     unsigned long long bytes = 0;
 };
 
 namespace {
 
+// Planes per chunk of member c.
 int member_kc(const r3d_ens_ctx* e, const r3d_hip_ctx* c) {
     if (e->tile.kc > 0) return std::min(e->tile.kc, c->cfg.npz);
     return std::min(32, c->cfg.npz);
@@ -280,15 +270,9 @@ void drop_graphs(r3d_ens_ctx* e) {
         }
 }
 
-// Threads of a persistent-launch block at the current tiling.
-int wave_count(int ty, int tw) { return tw == 64 ? ty + 3 : ty / (64 / tw) + 2; }
-int persistent_threads(const r3d_ens_ctx* e) { return wave_count(e->tile.ty, e->tile.tw) * 64; }
-
 // Rebuild the member table for the current tiling and parity.
 int build_table(r3d_ens_ctx* e) {
-    int tile0 = 0, bnd0 = 0;
-    const int npt = persistent_threads(e);
-    e->nbb_max = 0;
+    int tile0 = 0;
     for (size_t m = 0; m < e->mem.size(); ++m) {
         r3d_hip_ctx* c = e->mem[m];
         EnsMember& d = e->desc[m];
@@ -298,24 +282,21 @@ int build_table(r3d_ens_ctx* e) {
         for (int f = 0; f < NXF; ++f) d.z.q[f] = c->z[f];
         d.partial = e->part[m];
         d.scal = c->scal;
+        StagePlan pl{};
+        chunks_of(pl, c->cfg.npz, member_kc(e, c));
         d.ntx = (c->cfg.npx + e->tile.tw - 1) / e->tile.tw;
         d.nty = (c->cfg.npy + e->tile.ty - 1) / e->tile.ty;
-        d.kc = member_kc(e, c);
-        d.nkc = (c->cfg.npz + d.kc - 1) / d.kc;
+        d.nkc = pl.nkc;
+        d.kq = pl.kq;
+        d.krem = pl.krem;
         d.nblocks = d.ntx * d.nty * d.nkc;
-        d.nbb = c->nbb;
         d.tile0 = tile0;
         d.npart_dt = ENS_DT_BLOCKS;
-        d.nbbp = ((c->cfg.npx + 2) * (c->cfg.npy + 2) + npt - 1) / npt;
-        d.bnd0 = bnd0;
-        bnd0 += 2 * d.nbbp;
         d.C = c->C;
         d.M = c->M;
         tile0 += d.nblocks;
-        e->nbb_max = std::max(e->nbb_max, d.nbb);
     }
     e->ntiles = tile0;
-    e->nbunits = bnd0;
     e->grid = (tile0 + 7) / 8 * 8;
     HIPCHK(hipMemcpyAsync(e->d_desc, e->desc.data(), e->desc.size() * sizeof(EnsMember),
                           hipMemcpyHostToDevice, e->stream));
@@ -352,17 +333,12 @@ int enqueue_step(r3d_ens_ctx* e, int cur) {
         else if (e->tile.ty == 8) launch_stages_ty<8, false>(e, s, cur);
         else launch_stages_ty<9, false>(e, s, cur);
         HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_bound_ens, dim3(e->nbb_max, 2, n), dim3(BOUND_THREADS), 0, e->stream,
-                           e->d_desc, cur, s);
-        HIPCHK(hipGetLastError());
         cur ^= 1;
     }
     hipLaunchKernelGGL(k_finish_ens, dim3(n), dim3(1024), 0, e->stream, e->d_desc, 1, 1);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_dt_redo_ens, dim3(ENS_DT_BLOCKS, n), dim3(DT_THREADS), 0, e->stream,
                        e->d_desc, cur);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_finish_redo_ens, dim3(n), dim3(1024), 0, e->stream, e->d_desc);
     HIPCHK(hipGetLastError());
     return R3D_OK;
 }
@@ -384,10 +360,10 @@ int launch_persistent_ty(r3d_ens_ctx* e, int nsteps) {
         return set_err(R3D_EUNSUP, "persistent ensemble: %d resident blocks of %d threads", nblk,
                        NT);
     const EnsMember* d = e->d_desc;
-    int nmem = (int)e->mem.size(), ntiles = e->ntiles, nbu = e->nbunits, cur = e->cur, ns = nsteps;
+    int nmem = (int)e->mem.size(), ntiles = e->ntiles, cur = e->cur, ns = nsteps;
     int* work = e->d_work;
     HIPCHK(hipMemsetAsync(work, 0, 16 * sizeof(int), e->stream));
-    void* args[] = {(void*)&d, &nmem, &ntiles, &nbu, &cur, &ns, (void*)&work};
+    void* args[] = {(void*)&d, &nmem, &ntiles, &cur, &ns, (void*)&work};
     HIPCHK(hipLaunchCooperativeKernel(fn, dim3(nblk), dim3(NT), args, 0, e->stream));
     return R3D_OK;
 }
@@ -494,7 +470,7 @@ int r3d_ens_create(int nmembers, const r3d_hip_cfg* cfgs, r3d_ens_ctx** out) {
             std::max<long>((long)((cfgs[m].npx + 63) / 64) * ((cfgs[m].npy + 3) / 4),
                            (long)((cfgs[m].npx + 31) / 32) * ((cfgs[m].npy + 7) / 8)),
             (long)((cfgs[m].npx + 15) / 16) * ((cfgs[m].npy + 15) / 16));
-        const long worst = cols * ((cfgs[m].npz + 7) / 8) + 2L * c->nbb;
+        const long worst = cols * ((cfgs[m].npz + 7) / 8);
         double* p = nullptr;
         const size_t np = (size_t)std::max<long>(worst, ENS_DT_BLOCKS) * NPART;
         if (hipMalloc((void**)&p, np * sizeof(double)) != hipSuccess)

@@ -86,11 +86,6 @@ __global__ void k_global_copy(double* padded, double* dense, Geo g, int to_dense
 }
 
 // Kernels of one run over the device functions of r3d_aux.hpp.
-__global__ __launch_bounds__(BOUND_THREADS) void k_bound(const StageArgs a, const Consts C,
-                                                         const Metrics M, int partial_base) {
-    bound_block(a, C, M, partial_base, blockIdx.x, gridDim.x, blockIdx.y);
-}
-
 __global__ __launch_bounds__(DT_THREADS) void k_dt(const Geo g, const State s, const Consts C,
                                                    const Metrics M, double* partial) {
     dt_block(g, s, C, M, partial, blockIdx.x, gridDim.x);
@@ -102,20 +97,10 @@ __global__ __launch_bounds__(1024) void k_finish(DevScal* sc, const double* part
     finish_block(sc, partial, npart, C, reduce, advance, screened);
 }
 
-// The exact dt pass after a screened reduction that could not prove its
-// extrema (DevScal::dt_redo); every block returns at once otherwise.
 __global__ __launch_bounds__(DT_THREADS) void k_dt_redo(const Geo g, const State s,
                                                         const Consts C, const Metrics M,
-                                                        double* partial, const DevScal* sc) {
-    if (!sc->dt_redo) return;
-    dt_block(g, s, C, M, partial, blockIdx.x, gridDim.x);
-}
-__global__ __launch_bounds__(1024) void k_finish_redo(DevScal* sc, const double* partial,
-                                                      int npart, const Consts C) {
-    // all threads read the flag before the reduction's first barrier; thread
-    // 0 clears it after the last
-    if (!sc->dt_redo) return;
-    finish_block(sc, partial, npart, C, 1, 0, 0);
+                                                        double* partial, DevScal* sc) {
+    redo_block(g, s, C, M, partial, sc, blockIdx.x, gridDim.x);
 }
 
 // grid = (perimeter blocks, npz): planes 1..npz
@@ -735,6 +720,9 @@ int launch_stage(r3d_hip_ctx* c, int stage, int zmode, int want_dt) {
             if (ht && dn) launch_stage_kernel<8, false, true, true>(c, a, stage, zmode);
             else if (ht) launch_stage_kernel<8, false, true, false>(c, a, stage, zmode);
             else launch_stage_kernel<8, false, false, true>(c, a, stage, zmode);
+        } else if (c->ty == TILE_Y_SMALL) {
+            launch_stage_kernel<TILE_Y_SMALL, false, false, false, TILE_W_SMALL>(c, a, stage,
+                                                                                 zmode);
         } else if (c->ty == 8) {
             launch_stage_kernel<8, false>(c, a, stage, zmode);
         } else {
@@ -744,11 +732,6 @@ int launch_stage(r3d_hip_ctx* c, int stage, int zmode, int want_dt) {
     if (rc) return rc;
     if (fma_err != hipSuccess)
         return set_err(R3D_EHIP, "FMA stage launch: %s", hipGetErrorString(fma_err));
-    rc = timed(c, 1, [&] {
-        hipLaunchKernelGGL(k_bound, dim3(c->nbb, 2), dim3(BOUND_THREADS), 0, c->stream, a, c->C,
-                           c->M, c->nblocks);
-    });
-    if (rc) return rc;
     c->cur ^= 1;
     return R3D_OK;
 }
@@ -844,23 +827,18 @@ int r3d::step_one(r3d_hip_ctx* c, int nstages, double* const* keep, double* cons
     }
     rc = timed(c, 3, [&] {
         hipLaunchKernelGGL(k_finish, dim3(1), dim3(1024), 0, c->stream, c->scal, c->partial,
-                           c->nblocks + 2 * c->nbb, c->C, nstages == 3 ? 1 : 0, 1,
+                           c->nblocks, c->C, nstages == 3 ? 1 : 0, 1,
                            nstages == 3 ? 1 : 0);
     });
     if (rc) return rc;
     if (nstages == 3) {
         // the screened reduction's fallback: an exact pass over the new state
-        // when its extrema were not proven (both kernels exit at once if so)
+        // when its extrema were not proven (the blocks exit at once if so)
         State s;
         for (int f = 0; f < NXF; ++f) s.q[f] = c->xs[c->cur][f];
         rc = timed(c, 2, [&] {
             hipLaunchKernelGGL(k_dt_redo, dim3(DT_BLOCKS), dim3(DT_THREADS), 0, c->stream, c->g,
-                               s, c->C, c->M, c->partial, (const DevScal*)c->scal);
-        });
-        if (rc) return rc;
-        rc = timed(c, 3, [&] {
-            hipLaunchKernelGGL(k_finish_redo, dim3(1), dim3(1024), 0, c->stream, c->scal,
-                               c->partial, DT_BLOCKS, c->C);
+                               s, c->C, c->M, c->partial, c->scal);
         });
         if (rc) return rc;
     }
@@ -946,8 +924,8 @@ int r3d_hip_create(const r3d_hip_cfg* cfg, r3d_hip_ctx** out) {
     c->uploaded.assign((size_t)f.npey * f.npez, 0);
     fill_consts(c);
 
-    const StagePlan pl = plan_stage(f.npx, f.npy, f.npz, f.lmag != 0, feature, f.tile_rows,
-                                    f.zchunk, cus);
+    const StagePlan pl = plan_stage(f.npx, f.npy, f.npz, f.lmag != 0, feature, f.variant == 1,
+                                    f.tile_rows, f.zchunk, cus);
     c->ty = pl.ty;
     c->tw = pl.tw;
     c->ntx = pl.ntx;
@@ -958,7 +936,6 @@ int r3d_hip_create(const r3d_hip_cfg* cfg, r3d_hip_ctx** out) {
     c->nkc = pl.nkc;
     c->nblocks = c->ntx * c->nty * c->nkc;
     c->grid = (c->nblocks + 7) / 8 * 8;
-    c->nbb = ((f.npx + 2) * (f.npy + 2) + BOUND_THREADS - 1) / BOUND_THREADS;
 
     int rc = R3D_OK;
     auto fail = [&](int code) {
@@ -995,7 +972,7 @@ int r3d_hip_create(const r3d_hip_cfg* cfg, r3d_hip_ctx** out) {
         if (hipMemsetAsync(c->z[f2], 0, fe * sizeof(double), c->stream) != hipSuccess)
             return fail(set_err(R3D_EHIP, "hipMemset failed"));
     }
-    const size_t npart = std::max<size_t>((size_t)c->nblocks + 2 * c->nbb, DT_BLOCKS);
+    const size_t npart = std::max<size_t>((size_t)c->nblocks, DT_BLOCKS);
     if ((rc = dev_alloc(c, &c->partial, npart * NPART))) return fail(rc);
     {
         void* p = nullptr;
@@ -1406,9 +1383,11 @@ int r3d_hip_step_noalloc(r3d_hip_ctx* c, int nsteps, int nstages) {
     int rc = check_ready(c);
     if (rc) return rc;
     // every partial slot a step reads is written earlier in the same step
-    // (stage-3 tiles, both boundary sides, or the dt pass), so the array's
+    // (stage-3 tiles or the dt pass), so the array's
     // contents from an earlier call never reach a result
-    const size_t need = std::max<size_t>((size_t)c->nblocks + 2 * c->nbb, DT_BLOCKS) * NPART;
+    // (the limit also counts a slot per 256 cells of either wall plane)
+    const size_t nbb = ((size_t)(c->cfg.npx + 2) * (c->cfg.npy + 2) + 255) / 256;
+    const size_t need = std::max<size_t>((size_t)c->nblocks + 2 * nbb, DT_BLOCKS) * NPART;
     if (need > kNoallocScratchDoubles)
         return set_err(R3D_EINVAL,
                        "step_noalloc: this grid needs %zu doubles of dt partials; the static "

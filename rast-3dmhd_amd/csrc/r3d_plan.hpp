@@ -21,9 +21,16 @@ inline int hydro_tile_rows(int npy) {
 // waves, the first tiling; 4% slower at 252x252x512, kept as an override)
 constexpr int TILE_Y_MAG = 12, TILE_W_MAG = 32;
 constexpr int TILE_Y_MAG64 = 5;
+// Hydro tile of small grids: 4 rows of 16 columns, one flux wave and two halo
+// waves.
+constexpr int TILE_Y_SMALL = 4, TILE_W_SMALL = 16;
 // Columns of a stage tile of ty rows.
-inline int tile_width(bool lmag, int ty) { return lmag && ty == TILE_Y_MAG ? TILE_W_MAG : 64; }
+inline int tile_width(bool lmag, int ty) {
+    return lmag ? (ty == TILE_Y_MAG ? TILE_W_MAG : 64)
+                : (ty == TILE_Y_SMALL ? TILE_W_SMALL : 64);
+}
 constexpr int KC_MAX = 128;  // planes of a chunk at most (the z metrics a tile stages in LDS)
+constexpr int KC_MIN = 3;    // and at least (the walls' extrapolation reads three)
 
 // Tiles of ty rows x tw columns, ntx x nty of them; nkc z chunks: chunk kz has
 // kq planes, the first krem chunks one more, the last ends at npz.  kc: planes
@@ -41,18 +48,25 @@ inline StagePlan stage_tiles(int npx, int npy, bool lmag, int ty) {
     p.nty = (npy + ty - 1) / ty;
     return p;
 }
-// Chunks of kc planes, the last one shorter.
-inline void chunks_of(StagePlan& p, int npz, int kc) {
-    p.nkc = (npz + kc - 1) / kc;
-    p.kc = p.kq = kc;
-    p.krem = 0;
-}
 // nkc chunks of as equal size as they can be.
 inline void equal_chunks(StagePlan& p, int npz, int nkc) {
     p.nkc = nkc;
     p.kq = npz / nkc;
     p.krem = npz % nkc;
     p.kc = p.kq + (p.krem > 0);
+}
+// Chunks of kc planes (8 or more), the last one shorter; equal ones if it would
+// have fewer than three planes.
+inline void chunks_of(StagePlan& p, int npz, int kc) {
+    const int nkc = (npz + kc - 1) / kc, last = npz - (nkc - 1) * kc;
+    if (last < KC_MIN) {
+        equal_chunks(p, npz, nkc);
+    } else {
+        p.nkc = nkc;
+        p.kq = kc;
+        p.krem = 0;
+    }
+    p.kc = kc;
 }
 
 // Relative time of a stage launch.  One stage tile fills a CU (its waves take
@@ -65,14 +79,21 @@ inline void equal_chunks(StagePlan& p, int npz, int nkc) {
 // 100x70x90: 52.6 (0.94 rounds of 9; 10.5), 64.7 (1.97 of 5; 13), 80.5 (1.13
 // of 8; 19); hydro 64x64x128: 24.7 (1 of 4; 5.5), 33 (0.5 of 8; 9.5), 40.3
 // (4 of 1; 10).  A round of 9-row tiles takes 1.165 times one of 8-row tiles
-// (504x504x1024: 8.22 against 7.94 ms at equal coverage).
+// (504x504x1024: 8.22 against 7.94 ms at equal coverage).  A plane of the 4 x 16
+// tile, whose one flux wave has a SIMD to itself, takes 0.62 of an 8-row tile's,
+// as long as every tile has a CU: a step of 16x16x32 46 us (40 tiles) against 63,
+// of 32x32x64 48 (256 tiles) against 64; with more tiles than CUs they share
+// SIMDs (48x48x96: 69 us with 504 tiles, 61 with 192 of 8 rows).
 inline double stage_cost(const StagePlan& p, int cus) {
     const long rounds = (p.blocks() + cus - 1) / cus;
-    return (double)rounds * (p.kc + 1.5) * (p.ty == TILE_Y ? 1.165 : 1.0);
+    const bool small = p.tw == TILE_W_SMALL;
+    if (small && rounds > 1) return 1e300;
+    return (double)rounds * (p.kc + 1.5) * (p.ty == TILE_Y ? 1.165 : (small ? 0.62 : 1.0));
 }
 
 // The split of one run.  feature: heat loss, density diffusion, flux
-// relaxation or LREM, whose hydro kernels are built with 8-row tiles only.
+// relaxation or LREM, whose hydro kernels are built with 8-row tiles only; fma:
+// the contracted variant, built without the small tile.
 // tile_rows / zchunk: the caller's choice, 0 = the library's.
 //
 // The first choice is the largest chunk of 128, 64, 32, 16 or 8 planes that
@@ -80,10 +101,11 @@ inline double stage_cost(const StagePlan& p, int cus) {
 // split does better.  Otherwise it can leave the last round nearly empty
 // (288 tiles on 256 CUs) or spend a third of the time filling 8-plane chunks,
 // so every number of chunks is priced with stage_cost and the cheapest taken
-// if it promises 6% or more: the model's order is right to about 3%, and so
-// are two runs of one launch.
-inline StagePlan plan_stage(int npx, int npy, int npz, bool lmag, bool feature, int tile_rows,
-                            int zchunk, int cus) {
+// if it promises 3% or more (504x504x256, 4 rounds of 128 planes against 16 of
+// 32: promised 3.4%, measured 1.6%), with LMAG 6% (252x252x512, 4 rounds of 86
+// against 10.5 of 32: promised 5%, measured 0.6%).
+inline StagePlan plan_stage(int npx, int npy, int npz, bool lmag, bool feature, bool fma,
+                            int tile_rows, int zchunk, int cus) {
     const int ty0 = tile_rows ? tile_rows
                               : (lmag ? TILE_Y_MAG : (feature ? 8 : hydro_tile_rows(npy)));
     StagePlan first = stage_tiles(npx, npy, lmag, ty0);
@@ -97,12 +119,12 @@ inline StagePlan plan_stage(int npx, int npy, int npz, bool lmag, bool feature, 
     }
     if (first.kc == KC_MAX && first.blocks() >= 2048) return first;
     StagePlan best = first;
-    double least = 0.94 * stage_cost(first, cus);
-    const bool both = !tile_rows && !lmag && !feature;  // 8 or 9 rows
-    for (int ty : {ty0, both ? 17 - ty0 : 0}) {
+    double least = (lmag ? 0.94 : 0.97) * stage_cost(first, cus);
+    const bool free = !tile_rows && !lmag && !feature;  // 8 or 9 rows, or 4 x 16
+    for (int ty : {ty0, free ? 17 - ty0 : 0, free && !fma ? TILE_Y_SMALL : 0}) {
         if (!ty) continue;
         StagePlan p = stage_tiles(npx, npy, lmag, ty);
-        for (int nkc = (npz + KC_MAX - 1) / KC_MAX; nkc <= npz; ++nkc) {
+        for (int nkc = (npz + KC_MAX - 1) / KC_MAX; KC_MIN * nkc <= npz; ++nkc) {
             equal_chunks(p, npz, nkc);
             // beyond 16 rounds only the filling grows
             if (p.blocks() > 16L * cus && nkc > (npz + KC_MAX - 1) / KC_MAX) break;

@@ -4,7 +4,8 @@
 //     F  = FLUXES(X)                      reference src/fluxes.cpp:44-533
 //     X' = Z + gam_s dt F                 reference src/step.cpp:53-80
 //     Z' = X' + zeta_s dt F               reference src/step.cpp:83-110 (next stage's mix)
-// and, in the last stage, the per-cell dt limits of X' for the next step.
+// with BCON applied to X' on the two walls (src/bcon.cpp:12-141) and, in the
+// last stage, the per-cell dt limits of X' for the next step.
 //
 // Halo.  The reference refreshes ghost cells by a halo exchange after every
 // stage (src/communicate.cpp:70-169).  Here a virtual rank's ghost cells are
@@ -192,6 +193,60 @@ struct TileShape {
     static constexpr int NW = TW == 64 ? TY + 3 : NFW + 2;
 };
 
+// Where tile t of a launch lies and which cell of it this lane holds.
+template <int TY, int TW>
+struct TileCell {
+    int i0, j0, k0, k1;  // first cell of the tile, planes of its chunk
+    int wv, ln;          // wave and lane
+    int r, c;            // LDS row and column (column 1..TW inside the tile)
+    int gi, gj;          // the cell
+    int fw;              // the flux wave's slot for its running dt extrema
+    bool act, heavy, outp;  // holds a cell; computes fluxes; the cell is an output cell
+
+    TileCell() = default;
+    __device__ __forceinline__ TileCell(const StageArgs& a, int t) {
+        constexpr int ROWS = TileShape<TY, TW>::ROWS, NFW = TileShape<TY, TW>::NFW;
+        // x fastest: the tiles an XCD runs at the same time are x-neighbours
+        // (whole tile rows), whose x-halo columns lie in each other's cache lines
+        const int tx = t % a.ntx;
+        const int rem = t / a.ntx;
+        const int ty = rem % a.nty;
+        const int kz = rem / a.nty;
+        i0 = 1 + TW * tx;
+        j0 = 1 + TY * ty;
+        k0 = 1 + a.kq * kz + min(kz, a.krem);
+        k1 = min(a.g.npz, k0 + a.kq - 1 + (kz < a.krem ? 1 : 0));
+        // the wave index is uniform over the wave; from a scalar register, the
+        // role branch below is a scalar branch
+        wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        ln = threadIdx.x & 63;
+        if (TW == 64 ? wv < ROWS : wv <= NFW) {
+            if constexpr (TW == 64) {
+                r = wv;
+                c = ln + 1;
+            } else {  // RPW rows per wave; wave NFW holds the two y-halo rows
+                constexpr int RPW = TileShape<TY, TW>::RPW;
+                const int q = ln / TW;
+                r = wv < NFW ? 1 + RPW * wv + q : (q == 1 ? TY + 1 : 0);
+                c = ln % TW + 1;
+                act = wv < NFW || q < 2;  // y-halo wave: lanes past the two rows idle
+            }
+            gi = i0 + c - 1;
+            gj = j0 - 1 + r;
+            if constexpr (TW == 64) act = true;
+        } else {
+            act = ln < 2 * ROWS;
+            r = act ? (ln >> 1) : 0;
+            c = (ln & 1) ? TW + 1 : 0;
+            gi = (ln & 1) ? i0 + TW : i0 - 1;
+            gj = j0 - 1 + r;
+        }
+        heavy = TW == 64 ? (wv >= 1) && (wv <= TY) : wv < NFW;
+        fw = TW == 64 ? wv - 1 : wv;
+        outp = heavy && gi <= a.g.npx && gj <= a.g.npy;
+    }
+};
+
 // LDS of one stage tile.  The kernel that runs the tile declares it, so that
 // a persistent kernel can run the three stages in one allocation (a union).
 template <int TY, int STAGE, bool MAG, bool HEAT, bool DEN, int TW = 64>
@@ -230,17 +285,70 @@ struct StageLds {
     double scr_s[NSC];
 };
 
+// The boundary condition on one wall cell (reference src/bcon.cpp:12-141;
+// LREM's forms golden/fortran/3dmhdsub.f:2852-2952): the momenta and the
+// temperature of cell (i, j) on the top (side 0, k = 1) or bottom (side 1,
+// k = npz) plane from the updated values there (ro, tt) and one and two planes
+// in (suffix 1, 2).  RW = 0; the caller handles BZ.  Not contracted in any
+// variant.
+struct WallCell {
+    double ru, rv, tt;
+};
+__device__ __forceinline__ WallCell bcon_cell(const Consts& C, const Metrics& M, const Geo& g,
+                                              int side, int i, int j, double ro, double ro1,
+                                              double ro2, double ru1, double ru2, double rv1,
+                                              double rv2, double tt, double tt1, double tt2) {
+#pragma clang fp contract(off)
+    WallCell w;
+    w.ru = ro * (C.c43 * ru1 / ro1 - C.c13 * ru2 / ro2);
+    w.rv = ro * (C.c43 * rv1 / ro1 - C.c13 * rv2 / ro2);
+    if (side == 0) {
+        switch (C.top_mode) {
+            case TOP_GAUSS_T:
+                tt = 1.0 - (1.0 - C.tpr) * M.e1[i] / C.hh * M.e2[j] / C.hh;
+                break;
+            case TOP_GAUSS_FLUX:
+                tt = C.c43 * tt1 - C.c13 * tt2 -
+                     C.c23 * M.dz_top *
+                         (C.theta - (C.theta - C.tpr) * M.e1[i] / C.hh * M.e2[j] / C.hh);
+                break;
+            case TOP_CONST_T:  // LREM: TU (golden/fortran/3dmhdsub.f:2852-2853)
+                tt = C.lrem ? C.tu : 1.0;
+                if (!C.lrem && C.half_t && i <= (g.npx + 2) / 2) tt = 1.0 - C.tp;
+                break;
+            case TOP_CONST_FLUX:  // LREM: + DZTU (:2876-2879)
+                tt = C.lrem ? C.c43 * tt1 - C.c13 * tt2 + C.dztu
+                            : C.c43 * tt1 - C.c13 * tt2 - C.c23 * M.dz_top * C.theta;
+                break;
+            default:
+                break;
+        }
+    } else {
+        if (C.izcon == 0)
+            tt = C.tb;
+        else if (C.lrem)  // + DZTB (golden/fortran/3dmhdsub.f:2949-2952)
+            tt = C.c43 * tt1 - C.c13 * tt2 + C.dztb;
+        else
+            tt = C.c43 * tt1 - C.c13 * tt2 + C.c23 * M.dz_bot * C.theta / M.rkapa[g.npz];
+    }
+    w.tt = tt;
+    return w;
+}
+
 // One tile t (0 <= t < a.nblocks) of one RK stage; the caller maps blocks to
-// tiles and provides the LDS.  ZMODE: 0 = Z' is the next stage's mix, 1 = Z
+// tiles and provides the LDS.  Returns whether the tile is on a wall
+// (stage_walls finishes it then), the lane's cell and, in the last stage, its dt
+// extrema in pm.  ZMODE: 0 = Z' is the next stage's mix, 1 = Z
 // keeps the saved state (a step truncated after stage 1), 2 = Z is not
 // written (last stage).
 // HEAT: the ITCON=2 embedded heat loss term is added to FT; DEN: density
 // diffusion is added to FR.  Separate instantiations, so that the default
 // kernels carry none of their registers or LDS.
 template <int TY, int STAGE, int ZMODE, bool MAG, bool HEAT = false, bool DEN = false, int TW = 64>
-__device__ __forceinline__ void stage_tile(const StageArgs& a, const Consts& C, const Metrics& M,
+__device__ __forceinline__ bool stage_tile(const StageArgs& a, const Consts& C, const Metrics& M,
                                            const int t,
-                                           StageLds<TY, STAGE, MAG, HEAT, DEN, TW>& L) {
+                                           StageLds<TY, STAGE, MAG, HEAT, DEN, TW>& L,
+                                           double pm[NPART], TileCell<TY, TW>& cell) {
     using LT = StageLds<TY, STAGE, MAG, HEAT, DEN, TW>;
     constexpr int ROWS = LT::ROWS;
     constexpr int NW = LT::NW;
@@ -250,7 +358,6 @@ __device__ __forceinline__ void stage_tile(const StageArgs& a, const Consts& C, 
     constexpr int ZX_DEN = 0, ZX_HEAT = DEN ? 6 : 0;
     constexpr int NPM = LT::NPM;
     auto& sh = L.sh;
-    auto& red = L.red;
     auto& zm = L.zm;
     auto& zx = L.zx;
     auto& hgx_s = L.hgx_s;
@@ -265,49 +372,12 @@ __device__ __forceinline__ void stage_tile(const StageArgs& a, const Consts& C, 
         a.scal->dt = a.scal->dt_next;
         a.scal->umach = a.scal->umach_next;
     }
-    // x fastest: the tiles an XCD runs at the same time are x-neighbours
-    // (whole tile rows), whose x-halo columns lie in each other's cache lines
-    const int tx = t % a.ntx;
-    const int rem = t / a.ntx;
-    const int ty = rem % a.nty;
-    const int kz = rem / a.nty;
     const Geo g = a.g;
-    const int i0 = 1 + TW * tx, j0 = 1 + TY * ty;
-    const int k0 = 1 + a.kq * kz + min(kz, a.krem);
-    const int k1 = min(g.npz, k0 + a.kq - 1 + (kz < a.krem ? 1 : 0));
-
-    // the wave index is uniform over the wave; from a scalar register, the
-    // role branch below is a scalar branch
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
     constexpr int NFW = LT::NFW;
-    // LDS row and column of this lane (column 1..TW inside the tile)
-    int r, c, gi, gj;
-    bool act;
-    if (TW == 64 ? wv < ROWS : wv <= NFW) {
-        if constexpr (TW == 64) {
-            r = wv;
-            c = ln + 1;
-        } else {  // RPW rows per wave; wave NFW holds the two y-halo rows
-            constexpr int RPW = TileShape<TY, TW>::RPW;
-            const int q = ln / TW;
-            r = wv < NFW ? 1 + RPW * wv + q : (q == 1 ? TY + 1 : 0);
-            c = ln % TW + 1;
-            act = wv < NFW || q < 2;  // y-halo wave: lanes past the two rows idle
-        }
-        gi = i0 + c - 1;
-        gj = j0 - 1 + r;
-        if constexpr (TW == 64) act = true;
-    } else {
-        act = ln < 2 * ROWS;
-        r = act ? (ln >> 1) : 0;
-        c = (ln & 1) ? TW + 1 : 0;
-        gi = (ln & 1) ? i0 + TW : i0 - 1;
-        gj = j0 - 1 + r;
-    }
-    const bool heavy = TW == 64 ? (wv >= 1) && (wv <= TY) : wv < NFW;
-    // the flux wave's slot for its running dt extrema
-    const int fw = TW == 64 ? wv - 1 : wv;
-    const bool outp = heavy && gi <= g.npx && gj <= g.npy;
+    const TileCell<TY, TW> me(a, t);
+    const int i0 = me.i0, j0 = me.j0, k0 = me.k0, k1 = me.k1, r = me.r, c = me.c, wv = me.wv;
+    const int ln = me.ln, gi = me.gi, gj = me.gj, fw = me.fw;
+    const bool act = me.act, heavy = me.heavy, outp = me.outp;
     // the column this lane reads: periodic wrap at the x/y edges; lanes past
     // the wrap (partial edge tiles) read column/row 1 and their stores go to
     // the row padding
@@ -386,8 +456,6 @@ __device__ __forceinline__ void stage_tile(const StageArgs& a, const Consts& C, 
 
     Col cm = derive(rm);
     Col cc = derive(rc);
-
-    double pm[NPART] = {0.0, 1e300, 1e300, 1e300, 1e300};
 
     // The z loop is instantiated twice: for the flux rows (HEAVY) and for the
     // halo waves, which only load and publish.  Both run one barrier per
@@ -510,8 +578,8 @@ __device__ __forceinline__ void stage_tile(const StageArgs& a, const Consts& C, 
                 if (ZMODE == 1) {
                     stp(a.z.q[f], g.pp, k, soff, cur);
                 } else if (ZMODE == 0 && STAGE < 2) {
-                    // on the two BCON planes Z' holds F until the boundary
-                    // kernel mixes it with the post-BCON state
+                    // on the two BCON planes Z' holds F until it is mixed with
+                    // the post-BCON state, after the loop
                     stp(a.z.q[f], g.pp, k, soff, bplane ? fval : x + cz * fval);
                 }
             };
@@ -832,10 +900,98 @@ __device__ __forceinline__ void stage_tile(const StageArgs& a, const Consts& C, 
     else
         zloop(BoolConst<false>{});
 
-    if (STAGE == 2 && a.want_dt) {
-        if (heavy)
-            for (int q = 0; q < NPM; ++q) pm[q] = pmw_s[q][fw];
-        block_partials<NW>(pm, red, a.partial, t);
+    pm[0] = 0.0;
+    for (int q = 1; q < NPART; ++q) pm[q] = 1e300;
+    if (STAGE == 2 && a.want_dt && heavy)
+        for (int q = 0; q < NPM; ++q) pm[q] = pmw_s[q][fw];
+    cell = me;
+    return k0 == 1 || k1 == g.npz;
+}
+
+// The walls, after stage_tile, by the tiles whose chunk ends on one: BCON, the
+// deferred Z' mix there, in the last stage the wall cells' dt limits (into
+// pm), and the outer ghost plane.  Every chunk has three planes or more, so the
+// values BCON extrapolates from are this column's, stored by this lane in the z
+// loop; they are read back (a few cache hits a lane, in the tiles on a wall
+// only).  As a kernel of its own this pass cost 4 to 5 us a stage on small
+// grids (a step of 64x64x128: 89.0 us, now 75.7; MHD 100x70x90: 181, now 164),
+// and as much as it does here on large ones (504x504: 23 us a stage as a
+// kernel; here a wall tile's CU waits some 10 us, four times a launch).  The callers pass a, C and M by a second route, unrecognisable to the
+// compiler: what only this pass needs is then loaded here, and not held (and
+// spilled) across the z loop (1.5% at 504x504x256).
+template <int TY, int STAGE, int ZMODE, bool MAG, int TW>
+__device__ __forceinline__ void stage_walls(const StageArgs& a, const Consts& C, const Metrics& M,
+                                            const TileCell<TY, TW>& me, double pm[NPART]) {
+    constexpr int NF = MAG ? 8 : 5;
+    constexpr bool MIX = ZMODE == 0 && STAGE < 2;
+    const Geo g = a.g;
+    const int gi = me.gi, gj = me.gj;
+    const uint32_t voff = (uint32_t)((XOFF + gi + (long)g.px * gj) * 8);  // the true cell
+    // ghost cells of x and y: the halo lanes', and lanes past a partial tile's edge
+    const bool ghost = me.act && gi >= 0 && gj >= 0 && gi <= g.npx + 1 && gj <= g.npy + 1 &&
+                       (gi == 0 || gi == g.npx + 1 || gj == 0 || gj == g.npy + 1);
+    if (!me.outp && !ghost) return;
+    for (int side = 0; side < 2; ++side) {
+        if (side ? me.k1 != g.npz : me.k0 != 1) continue;
+        const int ko = side ? g.npz + 1 : 0, kb = side ? g.npz : 1, d = side ? -1 : 1;
+        // Every load first: the tile has its CU to itself, so that nothing else
+        // covers their latency, and past a store the compiler would wait.
+        const double rout = ldp(a.xin.q[QRO], g.pp, ko, voff);
+        double x[NF][3], z[NF], met[3] = {0.0, 0.0, 0.0};
+        if (me.outp) {
+            for (int f = 0; f < NF; ++f) {
+                if (f == QRW) continue;
+                x[f][0] = ldp(a.xout.q[f], g.pp, kb, voff);
+                if (f > QTT) continue;
+                x[f][1] = ldp(a.xout.q[f], g.pp, kb + d, voff);
+                x[f][2] = ldp(a.xout.q[f], g.pp, kb + 2 * d, voff);
+            }
+            if constexpr (MIX)
+                for (int f = 0; f < NF; ++f) z[f] = ldp(a.z.q[f], g.pp, kb, voff);
+            if (STAGE == 2) {
+                met[0] = dmin(dmin(M.ddx[gi], M.ddy[gj]), M.ddz[kb]);
+                met[1] = M.rkdt[kb];
+            }
+        }
+        // the step's dt (stage 1 of another tile may not have stored it yet)
+        const double cz = MIX ? C.zeta[STAGE < 2 ? STAGE : 0] *
+                                    (STAGE == 0 ? a.scal->dt_next : a.scal->dt)
+                              : 0.0;
+        // The outer ghost plane: the reference's FLUXES inverts RO on its full
+        // array (src/fluxes.cpp:133-138), x and y ghosts included, and its halo
+        // exchange never refreshes this plane.
+        stp(a.xout.q[QRO], g.pp, ko, voff, 1.0 / rout);
+        if (!me.outp) continue;
+        const double ro = x[QRO][0];
+        const WallCell w =
+            bcon_cell(C, M, g, side, gi, gj, ro, x[QRO][1], x[QRO][2], x[QRU][1], x[QRU][2],
+                      x[QRV][1], x[QRV][2], x[QTT][0], x[QTT][1], x[QTT][2]);
+        double y[NF];  // the post-BCON state
+        y[QRU] = w.ru;
+        y[QRV] = w.rv;
+        y[QRW] = 0.0;
+        y[QRO] = ro;
+        y[QTT] = w.tt;
+        if constexpr (MAG) {
+            // BZ = 0 on both walls (src/bcon.cpp:95-98, 136-139); BX, BY keep
+            // their updated values
+            y[QBX] = x[QBX][0];
+            y[QBY] = x[QBY][0];
+            y[QBZ] = C.bz_zero ? 0.0 : x[QBZ][0];
+        }
+        for (int f = 0; f < NF; ++f) {
+            if (f != QRO && f != QBX && f != QBY) stp(a.xout.q[f], g.pp, kb, voff, y[f]);
+            if constexpr (MIX) {  // the loop left F in Z
+#pragma clang fp contract(off)
+                stp(a.z.q[f], g.pp, kb, voff, y[f] + cz * z[f]);
+            }
+        }
+        if (STAGE == 2 && a.want_dt) {
+            double b[3] = {0.0, 0.0, 0.0};
+            if constexpr (MAG)
+                for (int q = 0; q < 3; ++q) b[q] = y[QBX + q];
+            dt_terms<MAG>(C, w.ru, w.rv, 0.0, ro, w.tt, b[0], b[1], b[2], met[0], met[1], pm);
+        }
     }
 }
 
@@ -847,7 +1003,22 @@ __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_stage(const St
     __shared__ StageLds<TY, STAGE, MAG, HEAT, DEN, TW> lds;
     const int t = logical_block();
     if (t >= a.nblocks) return;
-    stage_tile<TY, STAGE, ZMODE, MAG, HEAT, DEN, TW>(a, C, M, t, lds);
+    double pm[NPART];
+    TileCell<TY, TW> me;
+    if (stage_tile<TY, STAGE, ZMODE, MAG, HEAT, DEN, TW>(a, C, M, t, lds, pm, me)) {
+        struct Args {  // the arguments once more, from the kernel's argument segment
+            StageArgs a;
+            Consts C;
+            Metrics M;
+        };
+        auto* k =
+            (const __attribute__((address_space(4))) Args*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(k));
+        const Args& w = *(const Args*)k;
+        stage_walls<TY, STAGE, ZMODE, MAG, TW>(w.a, w.C, w.M, me, pm);
+    }
+    if (STAGE == 2 && a.want_dt)
+        block_partials<TileShape<TY, TW>::NW>(pm, lds.red, a.partial, t);
 }
 
 }  // namespace R3D_KNS

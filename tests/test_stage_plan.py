@@ -1,7 +1,9 @@
 """The stage kernel's split into tiles and z chunks (r3d_plan.hpp), on the CPU.
 
-Over a wide range of grids the planned chunks cover every plane once and fit
-the 128 planes of z metrics a tile stages, no split has more than 32 times
+Over a wide range of grids the planned chunks cover every plane once, have at
+least the three planes the walls' extrapolation reads and fit the 128 planes
+of z metrics a tile stages, the small tile is taken only where every tile has a
+CU (and not by the contracted variant, which is built without it), no split has more than 32 times
 as many tiles as CUs unless the grid needs them at 128-plane chunks, forced
 tilings are taken as given, and r3d_hip_step_noalloc's static scratch (131072
 doubles, five per tile and boundary block) accepts exactly the grids it
@@ -24,7 +26,7 @@ static bool covers(const StagePlan& p, int npz) {
         const int k0 = 1 + p.kq * kz + (kz < p.krem ? kz : p.krem);
         int k1 = k0 + p.kq - 1 + (kz < p.krem ? 1 : 0);
         if (k1 > npz) k1 = npz;
-        if (k0 != next || k1 < k0 || k1 - k0 + 1 > KC_MAX || k1 - k0 + 1 > p.kc) return false;
+        if (k0 != next || k1 < k0 || k1 - k0 + 1 > KC_MAX || k1 - k0 + 1 < KC_MIN || k1 - k0 + 1 > p.kc) return false;
         next = k1 + 1;
     }
     return next == npz + 1;
@@ -35,7 +37,7 @@ int main(int argc, char** argv) {
     for (int x = 3; x <= 2600; x = x * 4 / 3 + 1)
         for (int y = 3; y <= 2600; y = y * 5 / 4 + 1)
             for (int z = 6; z <= 6000; z = z * 9 / 8 + 1, ++n) {
-                const StagePlan p = plan_stage(x, y, z, lmag, feature, 0, 0, 256);
+                const StagePlan p = plan_stage(x, y, z, lmag, feature, false, 0, 0, 256);
                 StagePlan o = stage_tiles(x, y, lmag, lmag ? TILE_Y_MAG : feature ? 8 : hydro_tile_rows(y));
                 for (int kc : {128, 64, 32, 16, 8}) {
                     chunks_of(o, z, kc);
@@ -46,10 +48,12 @@ int main(int argc, char** argv) {
                 const bool is = (p.blocks() + 2 * nbb) * 5 <= 131072;
                 const bool ok = covers(p, z) && was == is && stage_cost(p, 256) <= stage_cost(o, 256) &&
                                 (p.blocks() <= 32 * 256 || p.blocks() == o.blocks()) &&
-                                (!feature || lmag || p.ty == 8);
+                                (!feature || lmag || p.ty == 8) &&
+                                (p.tw != TILE_W_SMALL || p.blocks() <= 256) &&
+                                plan_stage(x, y, z, lmag, feature, true, 0, 0, 256).tw != TILE_W_SMALL;
                 if (!ok && bad++ < 5) printf("%d x %d x %d: ty %d kc %d nkc %d\n", x, y, z, p.ty, p.kc, p.nkc);
                 for (int kc : {8, 128}) {
-                    const StagePlan f = plan_stage(x, y, z, lmag, feature, o.ty, kc, 256);
+                    const StagePlan f = plan_stage(x, y, z, lmag, feature, false, o.ty, kc, 256);
                     if (!covers(f, z) || f.kc != kc || f.ty != o.ty) ++bad;
                 }
             }
