@@ -187,7 +187,7 @@ int r3d_hip_sync(r3d_hip_ctx* ctx);
 /* Kernel timing: when enabled, each stage launch is bracketed by HIP events
  * on the context stream; r3d_hip_kernel_stats returns, per kernel class
  * (0 = fused stage kernel, the boundary conditions included, 1 = none: the
- * boundary kernel it once was, 2 = dt kernel, 3 = small kernels), the number of
+ * boundary kernel it once was, 2 = dt kernel, 3 = the step's closing reduction), the number of
  * launches and their total milliseconds since the last reset. */
 int r3d_hip_set_timing(r3d_hip_ctx* ctx, int enable);
 int r3d_hip_kernel_stats(r3d_hip_ctx* ctx, int cls, long* launches, double* total_ms);

@@ -5,6 +5,8 @@
 // k_dt      : dt limits of the current state when no fused value is
 //             available (first step, after an upload or a truncated step).
 // k_finish  : reduces the dt partials and advances the step counters.
+// k_finish_redo: the same at the end of a step of few tiles, with the exact
+//             pass over the limits where the screened ones prove nothing.
 #pragma once
 
 #include "r3d_stage.hpp"
@@ -63,6 +65,49 @@ __device__ __forceinline__ void halo_thread(const Geo& g, const State& x, int nf
     for (int f = 0; f < nf; ++f) x.q[f][d] = x.q[f][s];
 }
 
+// The extrema of partial[0..npart), in thread 0 of a block of NT.
+template <int NT>
+__device__ __forceinline__ void reduce_partials(const double* partial, int npart, double* o) {
+    __shared__ double red[NT / 64][NPART];
+    double pm[NPART] = {0.0, 1e300, 1e300, 1e300, 1e300};
+    for (int q = threadIdx.x; q < npart; q += NT) {
+        pm[0] = dmax(pm[0], partial[(long)q * NPART]);
+        for (int v = 1; v < NPART; ++v) pm[v] = dmin(pm[v], partial[(long)q * NPART + v]);
+    }
+    const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
+    double v[NPART];
+    v[0] = wave_max(pm[0]);
+    for (int q = 1; q < NPART; ++q) v[q] = wave_min(pm[q]);
+    if (ln == 0)
+        for (int q = 0; q < NPART; ++q) red[wv][q] = v[q];
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int q = 0; q < NPART; ++q) o[q] = red[0][q];
+    for (int w = 1; w < NT / 64; ++w) {
+        o[0] = dmax(o[0], red[w][0]);
+        for (int q = 1; q < NPART; ++q) o[q] = dmin(o[q], red[w][q]);
+    }
+}
+
+__device__ __forceinline__ double least_limit(const Consts& C, const double* o) {
+    const double m = dmin(dmin(o[1], o[2]), o[3]);
+    return C.lmag ? dmin(m, o[4]) : m;
+}
+
+__device__ __forceinline__ void advance_counters(DevScal* sc) {
+    sc->nit += 1;
+    sc->timc += sc->dt;
+    sc->timt = sc->timi + sc->timc;
+}
+
+// The next step's dt and umach from the extrema m and um.
+__device__ __forceinline__ void set_next(DevScal* sc, const Consts& C, double m, double um) {
+    sc->umach_next = sqrt(um);
+    sc->dt_next = C.dtfix > 0.0 ? C.dtfix : C.sff * m;
+    sc->lim_next = m;
+    sc->um_next = um;
+}
+
 // One block of NT threads.  reduce: fold partial[0..npart) into dt_next /
 // umach_next (dt = sff * min of the limits, src/step.cpp:224-229; umach =
 // sqrt(max), src/step.cpp:141).  advance: the end-of-step counters
@@ -77,58 +122,24 @@ template <int NT = 1024>
 __device__ __forceinline__ void finish_block(DevScal* sc, const double* partial, int npart,
                                              const Consts& C, int reduce, int advance,
                                              int screened = 0) {
-    __shared__ double red[NT / 64][NPART];
-    double pm[NPART] = {0.0, 1e300, 1e300, 1e300, 1e300};
-    if (reduce)
-        for (int q = threadIdx.x; q < npart; q += NT) {
-            pm[0] = dmax(pm[0], partial[(long)q * NPART]);
-            for (int v = 1; v < NPART; ++v) pm[v] = dmin(pm[v], partial[(long)q * NPART + v]);
-        }
-    const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
-    double v[NPART];
-    v[0] = wave_max(pm[0]);
-    for (int q = 1; q < NPART; ++q) v[q] = wave_min(pm[q]);
-    if (ln == 0)
-        for (int q = 0; q < NPART; ++q) red[wv][q] = v[q];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        if (advance) {
-            sc->nit += 1;
-            sc->timc += sc->dt;
-            sc->timt = sc->timi + sc->timc;
-        }
-        if (reduce) {
-            double o[NPART];
-            for (int q = 0; q < NPART; ++q) o[q] = red[0][q];
-            for (int w = 1; w < NT / 64; ++w) {
-                o[0] = dmax(o[0], red[w][0]);
-                for (int q = 1; q < NPART; ++q) o[q] = dmin(o[q], red[w][q]);
-            }
-            double m = dmin(dmin(o[1], o[2]), o[3]);
-            if (C.lmag) m = dmin(m, o[4]);
-            const bool proven =
-                !screened || screen_proven(C, m, o[0], sc->lim_prev, sc->um_prev);
-            sc->dt_redo = proven ? 0 : 1;
-            if (proven) {
-                sc->umach_next = sqrt(o[0]);
-                sc->dt_next = C.dtfix > 0.0 ? C.dtfix : C.sff * m;
-                sc->lim_prev = m;
-                sc->um_prev = o[0];
-            }
-        }
+    double o[NPART];
+    reduce_partials<NT>(partial, reduce ? npart : 0, o);
+    if (threadIdx.x != 0) return;
+    if (advance) advance_counters(sc);
+    if (reduce) {
+        const double m = least_limit(C, o);
+        const bool proven = !screened || screen_proven(C, m, o[0], sc->lim_prev, sc->um_prev);
+        sc->dt_redo = proven ? 0 : 1;
+        if (proven) set_next(sc, C, m, o[0]);
     }
 }
 
-// The exact dt pass after a screened reduction that could not prove its
-// extrema (DevScal::dt_redo): block bx of nbx reduces its share of the state,
-// and the block that ends last reduces the partials (both in one launch, which
-// costs a step 2 us when there is nothing to do).  Every thread reads the
-// flag at its block's start; the last block clears it, when all have started.
-template <int NT = DT_THREADS>
-__device__ __forceinline__ void redo_block(const Geo& g, const State& s, const Consts& C,
+// The limits of the whole state, block bx of nbx; the block that ends last
+// reduces the partials and records the extrema.
+template <int NT>
+__device__ __forceinline__ void exact_pass(const Geo& g, const State& s, const Consts& C,
                                            const Metrics& M, double* partial, DevScal* sc, int bx,
                                            int nbx) {
-    if (!sc->dt_redo) return;
     __shared__ int last;
     dt_block<NT>(g, s, C, M, partial, bx, nbx);
     if (threadIdx.x == 0) {
@@ -140,6 +151,45 @@ __device__ __forceinline__ void redo_block(const Geo& g, const State& s, const C
     __threadfence();  // the other blocks' partials
     finish_block<NT>(sc, partial, nbx, C, 1, 0, 0);
     if (threadIdx.x == 0) sc->redo_done = 0;
+}
+
+// The exact dt pass after a screened reduction that could not prove its
+// extrema (DevScal::dt_redo): block bx of nbx reduces its share of the state,
+// and the block that ends last reduces the partials (both in one launch, which
+// costs a step 2 us when there is nothing to do).  Every thread reads the
+// flag at its block's start; the last block clears it, when all have started.
+template <int NT = DT_THREADS>
+__device__ __forceinline__ void redo_block(const Geo& g, const State& s, const Consts& C,
+                                           const Metrics& M, double* partial, DevScal* sc, int bx,
+                                           int nbx) {
+    if (sc->dt_redo) exact_pass<NT>(g, s, C, M, partial, sc, bx, nbx);
+}
+
+// finish_block of a screened step and redo_block in one launch: every block
+// reduces the partials for itself and knows whether they prove the extrema; if
+// so block 0 records them, else all take the exact pass.  The screen's
+// thresholds stay as they are until the next step's stage 1, the exact pass has
+// its own partials behind the stage's, and its last block records, so nothing
+// that a block reads is written by another.
+template <int NT>
+__device__ __forceinline__ void finish_redo_block(const Geo& g, const State& s, const Consts& C,
+                                                  const Metrics& M, double* partial, int npart,
+                                                  double* exact, DevScal* sc, int bx, int nbx) {
+    __shared__ int flag;
+    double o[NPART];
+    reduce_partials<NT>(partial, npart, o);
+    if (threadIdx.x == 0) {
+        const double m = least_limit(C, o);
+        const bool proven = screen_proven(C, m, o[0], sc->lim_prev, sc->um_prev);
+        if (bx == 0) {
+            advance_counters(sc);
+            if (proven) set_next(sc, C, m, o[0]);
+        }
+        flag = proven;
+    }
+    __syncthreads();
+    if (flag) return;
+    exact_pass<NT>(g, s, C, M, exact, sc, bx, nbx);
 }
 
 }  // namespace R3D_KNS

@@ -16,6 +16,15 @@
 namespace r3d {
 
 constexpr int DT_BLOCKS = 1024;
+// Blocks of the launch that ends a step: each reduces all of the stage's
+// partials (at most 30 KB) and takes its share of the exact pass if they prove
+// nothing; taken where the pass's own partials fit behind the stage's among the
+// DT_BLOCKS slots.  4.5 to 5 us, where a block's reduction and a launch of
+// blocks that exit took 5.8 and 2 to 5: a step of 16x16x32 45.5 -> 42.0 us,
+// 64x64x128 81.0 -> 77.5, MHD 100x70x90 184 -> 180.  With more tiles than that
+// the two launches stay: the blocks would read the partials 256 times over, and
+// the 5 us are less than a thousandth of such a step.
+constexpr int FIN_BLOCKS = 256, FIN_THREADS = 512;
 
 // Set the calling thread's error message and return code.
 int set_err(int code, const char* fmt, ...);

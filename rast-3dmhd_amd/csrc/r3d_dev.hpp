@@ -36,9 +36,11 @@ struct DevScal {
     double dt, timc, timt, timi, umach;
     double dt_next, umach_next;
     int nit, pad;
-    // the last reduction's extrema: the least time-step limit over all cells
-    // and limits, and the largest ogamma*UU/T; they set the next screen (below)
+    // the extrema of the reduction that gave dt: the least time-step limit over
+    // all cells and limits, and the largest ogamma*UU/T; they set the screen of
+    // the step's stage 3 (below).  Stage 1 takes them, like dt, from *_next.
     double lim_prev, um_prev;
+    double lim_next, um_next;
     int dt_redo;    // the screened reduction could not prove its extrema: redo exactly
     int redo_done;  // blocks of that exact pass that have written their partial
 };

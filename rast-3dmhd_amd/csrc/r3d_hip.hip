@@ -103,6 +103,14 @@ __global__ __launch_bounds__(DT_THREADS) void k_dt_redo(const Geo g, const State
     redo_block(g, s, C, M, partial, sc, blockIdx.x, gridDim.x);
 }
 
+__global__ __launch_bounds__(FIN_THREADS) void k_finish_redo(const Geo g, const State s,
+                                                             const Consts C, const Metrics M,
+                                                             double* partial, int npart,
+                                                             DevScal* sc) {
+    finish_redo_block<FIN_THREADS>(g, s, C, M, partial, npart, partial + (long)npart * NPART, sc,
+                                   blockIdx.x, gridDim.x);
+}
+
 // grid = (perimeter blocks, npz): planes 1..npz
 __global__ __launch_bounds__(HALO_THREADS) void k_halo(const Geo g, const State x, int nf) {
     halo_thread(g, x, nf, blockIdx.x * HALO_THREADS + threadIdx.x, 1 + blockIdx.y);
@@ -825,6 +833,16 @@ int r3d::step_one(r3d_hip_ctx* c, int nstages, double* const* keep, double* cons
                 HIPCHK(hipMemcpyAsync(keep[s] + f * fe, c->xs[c->cur][f], fe * sizeof(double),
                                       hipMemcpyDeviceToDevice, c->stream));
     }
+    State s;
+    for (int f = 0; f < NXF; ++f) s.q[f] = c->xs[c->cur][f];
+    if (nstages == 3 && c->nblocks + FIN_BLOCKS <= DT_BLOCKS) {
+        rc = timed(c, 3, [&] {
+            hipLaunchKernelGGL(k_finish_redo, dim3(FIN_BLOCKS), dim3(FIN_THREADS), 0, c->stream,
+                               c->g, s, c->C, c->M, c->partial, c->nblocks, c->scal);
+        });
+        c->next_valid = rc == R3D_OK;
+        return rc;
+    }
     rc = timed(c, 3, [&] {
         hipLaunchKernelGGL(k_finish, dim3(1), dim3(1024), 0, c->stream, c->scal, c->partial,
                            c->nblocks, c->C, nstages == 3 ? 1 : 0, 1,
@@ -834,8 +852,6 @@ int r3d::step_one(r3d_hip_ctx* c, int nstages, double* const* keep, double* cons
     if (nstages == 3) {
         // the screened reduction's fallback: an exact pass over the new state
         // when its extrema were not proven (the blocks exit at once if so)
-        State s;
-        for (int f = 0; f < NXF; ++f) s.q[f] = c->xs[c->cur][f];
         rc = timed(c, 2, [&] {
             hipLaunchKernelGGL(k_dt_redo, dim3(DT_BLOCKS), dim3(DT_THREADS), 0, c->stream, c->g,
                                s, c->C, c->M, c->partial, c->scal);

@@ -371,6 +371,8 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, const Consts& C, 
     if (STAGE == 0 && t == 0 && threadIdx.x == 0) {
         a.scal->dt = a.scal->dt_next;
         a.scal->umach = a.scal->umach_next;
+        a.scal->lim_prev = a.scal->lim_next;
+        a.scal->um_prev = a.scal->um_next;
     }
     const Geo g = a.g;
     constexpr int NFW = LT::NFW;
