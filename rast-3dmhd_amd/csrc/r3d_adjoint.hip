@@ -223,21 +223,34 @@ __global__ __launch_bounds__(AT) void k_bcon_adj(const Geo g, const State X, con
         const long n = g.at(i, j, kw);
         const long d1 = side ? -g.pp : g.pp;
         const long n1 = n + d1, n2 = n + 2 * d1;
+        // all loads first: 5.9 us a launch at 128x128; as chains of loads,
+        // divisions and stores one after the other it took 10
         const double ro = X.q[QRO][n], ro1 = X.q[QRO][n1], ro2 = X.q[QRO][n2];
+        double m1[2], m2[2], l0[2], l1[2], l2[2];
+        for (int f = QRU; f <= QRV; ++f) {
+            m1[f] = X.q[f][n1];
+            m2[f] = X.q[f][n2];
+            l0[f] = LX.q[f][n];
+            l1[f] = LX.q[f][n1];
+            l2[f] = LX.q[f][n2];
+        }
+        double r0 = LX.q[QRO][n], r1 = LX.q[QRO][n1], r2 = LX.q[QRO][n2];
+        const double aT = LX.q[QTT][n], t1 = LX.q[QTT][n1], t2 = LX.q[QTT][n2];
         for (int f = QRU; f <= QRV; ++f) {
             // m = ro * (c43 m1 / ro1 - c13 m2 / ro2)  (src/bcon.cpp:22-37)
-            const double a = LX.q[f][n];
-            const double m1 = X.q[f][n1], m2 = X.q[f][n2];
-            LX.q[QRO][n] += a * (C.c43 * m1 / ro1 - C.c13 * m2 / ro2);
-            LX.q[f][n1] += a * ro * C.c43 / ro1;
-            LX.q[QRO][n1] -= a * ro * C.c43 * m1 / (ro1 * ro1);
-            LX.q[f][n2] -= a * ro * C.c13 / ro2;
-            LX.q[QRO][n2] += a * ro * C.c13 * m2 / (ro2 * ro2);
+            const double a = l0[f];
+            r0 += a * (C.c43 * m1[f] / ro1 - C.c13 * m2[f] / ro2);
+            LX.q[f][n1] = l1[f] + a * ro * C.c43 / ro1;
+            r1 -= a * ro * C.c43 * m1[f] / (ro1 * ro1);
+            LX.q[f][n2] = l2[f] - a * ro * C.c13 / ro2;
+            r2 += a * ro * C.c13 * m2[f] / (ro2 * ro2);
             LX.q[f][n] = 0.0;
         }
+        LX.q[QRO][n] = r0;
+        LX.q[QRO][n1] = r1;
+        LX.q[QRO][n2] = r2;
         LX.q[QRW][n] = 0.0;
         if (C.lmag && C.bz_zero) LX.q[QBZ][n] = 0.0;  // BZ = 0 on the walls
-        const double aT = LX.q[QTT][n];
         bool fixed = false, extrap = false;
         double dth = 0.0;
         if (side == 0) {
@@ -265,14 +278,15 @@ __global__ __launch_bounds__(AT) void k_bcon_adj(const Geo g, const State X, con
             dth = C.c23 * M.dz_bot / M.rkapa[kw];
         }
         if (extrap) {
-            LX.q[QTT][n1] += C.c43 * aT;
-            LX.q[QTT][n2] -= C.c13 * aT;
+            LX.q[QTT][n1] = t1 + C.c43 * aT;
+            LX.q[QTT][n2] = t2 - C.c13 * aT;
             gth = aT * dth;
         }
         if (fixed || extrap) LX.q[QTT][n] = 0.0;
     }
-    block_sum(gth, red, &acc[3]);
-    block_sum(gtb, red, &acc[5]);
+    if (side == 1 && C.izcon == 0) block_sum(gtb, red, &acc[5]);
+    else if (side == 1 || C.top_mode == TOP_GAUSS_FLUX || C.top_mode == TOP_CONST_FLUX)
+        block_sum(gth, red, &acc[3]);
 }
 
 // Objective per block (deterministic host sum) and, if LX is given, its
@@ -326,100 +340,75 @@ __global__ __launch_bounds__(AT) void k_ke(const Geo g, const State X, const Met
     }
 }
 
-// Per-block minimum of the dt limits (the formulas of dt_terms) with the key
-// cell * 4 + limit, ties to the smaller key.
-__global__ __launch_bounds__(AT) void k_dt_argmin(const Geo g, const State X, const Consts C,
-                                                  const Metrics M, double* bval, long* bkey) {
+// The least of the dt limits (the formulas of dt_terms) so far, with the key
+// cell * 4 + limit + 1, ties to the smaller key.
+struct LeastLimit {
+    double best = 1e300;
+    long key = LONG_MAX;
+    __device__ __forceinline__ void take(double v, long k) {
+        if (v < best || (v == best && k < key)) {
+            best = v;
+            key = k;
+        }
+    }
+};
+__device__ __forceinline__ void take_cell(const Geo& g, const State& X, const Consts& C,
+                                          const Metrics& M, long q, LeastLimit& m) {
     // the limits must round as the forward's dt reduction does, so that the
     // minimum falls on the same cell and limit
 #pragma clang fp contract(off)
-    __shared__ double rv[AT / 64];
-    __shared__ long rk[AT / 64];
-    double best = 1e300;
-    long key = LONG_MAX;
-    const long total = (long)g.npx * g.npy * g.npz;
-    for (long q = (long)blockIdx.x * AT + threadIdx.x; q < total; q += (long)gridDim.x * AT) {
-        int i, j, k;
-        cell_of(g, q, i, j, k);
-        const long n = g.at(i, j, k);
-        const double ru = X.q[QRU][n], rv_ = X.q[QRV][n], rw = X.q[QRW][n];
-        const double ro = X.q[QRO][n], tt = X.q[QTT][n];
-        const double dd = dmin(dmin(M.ddx[i], M.ddy[j]), M.ddz[k]);
-        const double uu = (ru * ru + rv_ * rv_ + rw * rw) * (1.0 / ro) * (1.0 / ro);
-        double fast;
-        if (C.lmag) {
-            const double bx = X.q[QBX][n], by = X.q[QBY][n], bz = X.q[QBZ][n];
-            const double b2 = (bx * bx + by * by + bz * bz) * C.obeta / ro;
-            fast = uu + C.gamma * tt + b2 + 2.0 * sqrt(uu * (C.gamma * tt + b2));
-        } else {
-            fast = uu + C.gamma * tt + 2.0 * sqrt(uu * C.gamma * tt);
-        }
-        const double L[4] = {dd / sqrt(fast), 0.5 * dd * dd * C.repr * C.cv * ro / M.rkapa[k],
-                             0.375 * dd * dd * C.re * ro, 0.5 * dd * dd * C.rm};
-        for (int t = 0; t < (C.lmag ? 4 : 3); ++t) {
-            const long kk = q * 4 + t + 1;
-            if (L[t] < best || (L[t] == best && kk < key)) {
-                best = L[t];
-                key = kk;
-            }
-        }
+    int i, j, k;
+    cell_of(g, q, i, j, k);
+    const long n = g.at(i, j, k);
+    const double ru = X.q[QRU][n], rv_ = X.q[QRV][n], rw = X.q[QRW][n];
+    const double ro = X.q[QRO][n], tt = X.q[QTT][n];
+    const double dd = dmin(dmin(M.ddx[i], M.ddy[j]), M.ddz[k]);
+    const double uu = (ru * ru + rv_ * rv_ + rw * rw) * (1.0 / ro) * (1.0 / ro);
+    double fast;
+    if (C.lmag) {
+        const double bx = X.q[QBX][n], by = X.q[QBY][n], bz = X.q[QBZ][n];
+        const double b2 = (bx * bx + by * by + bz * bz) * C.obeta / ro;
+        fast = uu + C.gamma * tt + b2 + 2.0 * sqrt(uu * (C.gamma * tt + b2));
+    } else {
+        fast = uu + C.gamma * tt + 2.0 * sqrt(uu * C.gamma * tt);
     }
+    const double L[4] = {dd / sqrt(fast), 0.5 * dd * dd * C.repr * C.cv * ro / M.rkapa[k],
+                         0.375 * dd * dd * C.re * ro, 0.5 * dd * dd * C.rm};
+    for (int t = 0; t < (C.lmag ? 4 : 3); ++t) m.take(L[t], q * 4 + t + 1);
+}
+// Over the block, in thread 0.
+__device__ __forceinline__ void block_least(LeastLimit& m) {
+    __shared__ double best[AT / 64];
+    __shared__ long key[AT / 64];
     for (int o = 32; o > 0; o >>= 1) {
-        const double ob = __shfl_xor(best, o, 64);
-        const long ok = __shfl_xor(key, o, 64);
-        if (ob < best || (ob == best && ok < key)) {
-            best = ob;
-            key = ok;
-        }
+        const double ob = __shfl_xor(m.best, o, 64);
+        const long ok = __shfl_xor(m.key, o, 64);
+        m.take(ob, ok);
     }
-    const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
-    if (ln == 0) {
-        rv[wv] = best;
-        rk[wv] = key;
+    if ((threadIdx.x & 63) == 0) {
+        best[threadIdx.x >> 6] = m.best;
+        key[threadIdx.x >> 6] = m.key;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < AT / 64; ++w)
-            if (rv[w] < best || (rv[w] == best && rk[w] < key)) {
-                best = rv[w];
-                key = rk[w];
-            }
-        bval[blockIdx.x] = best;
-        bkey[blockIdx.x] = key;
-    }
+    if (threadIdx.x == 0)
+        for (int w = 1; w < AT / 64; ++w) m.take(best[w], key[w]);
+    __syncthreads();
 }
 
-// Single block: the cell and limit attaining the minimum over the block
-// results, then LX[cell] += sff * lam_dt * dL/dX there, lam_dt = acc[2] / dt,
-// and acc[4] += sff * lam_dt * dL/dRe.  At a cell at rest the advective
-// limit's velocity derivative is taken as 0.
-__global__ __launch_bounds__(64) void k_dt_apply(const Geo g, const State X, const Consts C,
-                                                 const double* bval, const long* bkey, int nb,
-                                                 double dt, const State LX, double* acc) {
-    double best = 1e300;
-    long key = LONG_MAX;
-    for (int b = threadIdx.x; b < nb; b += 64)
-        if (bval[b] < best || (bval[b] == best && bkey[b] < key)) {
-            best = bval[b];
-            key = bkey[b];
-        }
-    for (int o = 32; o > 0; o >>= 1) {
-        const double ob = __shfl_xor(best, o, 64);
-        const long ok = __shfl_xor(key, o, 64);
-        if (ob < best || (ob == best && ok < key)) {
-            best = ob;
-            key = ok;
-        }
-    }
-    if (threadIdx.x != 0) return;
-    const long q = (key - 1) / 4;
-    const int t = (int)((key - 1) % 4);  // 0 advective, 1 thermal, 2 viscous
+// One thread: LX[cell] += sff * lam_dt * dL/dX at the cell and limit of the
+// minimum, lam_dt = acc[2] / dt, and acc[4] += sff * lam_dt * dL/dRe; acc[2]
+// is spent.  At a cell at rest the advective limit's velocity derivative is
+// taken as 0.
+__device__ void dt_apply(const Geo& g, const State& X, const Consts& C, const LeastLimit& m,
+                         double dt, const State& LX, double* acc) {
+    const long q = (m.key - 1) / 4;
+    const int t = (int)((m.key - 1) % 4);  // 0 advective, 1 thermal, 2 viscous
     int i, j, k;
     cell_of(g, q, i, j, k);
     const long n = g.at(i, j, k);
     const double ru = X.q[QRU][n], rv = X.q[QRV][n], rw = X.q[QRW][n];
     const double ro = X.q[QRO][n], tt = X.q[QTT][n];
-    const double L = best, s = C.sff * acc[2] / dt;
+    const double L = m.best, s = C.sff * acc[2] / dt;
     double dv[NXF] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, dre = 0.0;
     if (t == 0) {
         // L = dd / sqrt(fast), fast = uu + a + 2 sqrt(uu a), uu = |m|^2 / ro^2,
@@ -454,6 +443,50 @@ __global__ __launch_bounds__(64) void k_dt_apply(const Geo g, const State X, con
     }  // t = 3: the resistive limit 0.5 dd^2 Rm depends on neither
     for (int f = 0; f < (C.lmag ? 8 : 5); ++f) LX.q[f][n] += s * dv[f];
     acc[4] += s * dre;
+    acc[2] = 0.0;
+}
+
+// The adjoint of dt = sff * min of the limits.  The transpose of stage 1 has
+// listed the cells that may hold the minimum (cell[0 .. count[slot])): block 0
+// takes the exact limits of those.  With none or too many of them (a state at
+// rest, say) all blocks go over the whole state, and the one that ends last
+// reduces their results.  The steps use the two slots in turn, so that a count
+// is cleared while no block can read it.  At 128x128x256 8 us a step (MHD 11),
+// and the bounds some 15 of the transpose's 250 (443); the pass over the state
+// took 41 (56) at the copy rate of the card, its reduction by one wave 16 more.
+__global__ __launch_bounds__(AT) void k_dt_adj(const Geo g, const State X, const Consts C,
+                                               const Metrics M, const DtHits H, int* counts,
+                                               int slot, int* done, double* bval, long* bkey,
+                                               double dt, const State LX, double* acc) {
+    __shared__ int last;
+    const int n = counts[slot];
+    const long total = (long)g.npx * g.npy * g.npz;
+    LeastLimit m;
+    if (n >= 1 && n <= DT_HITS) {
+        if (blockIdx.x != 0) return;
+        for (int h = threadIdx.x; h < n; h += AT) take_cell(g, X, C, M, H.cell[h], m);
+        block_least(m);
+    } else {
+        for (long q = (long)blockIdx.x * AT + threadIdx.x; q < total; q += (long)gridDim.x * AT)
+            take_cell(g, X, C, M, q, m);
+        block_least(m);
+        if (threadIdx.x == 0) {
+            bval[blockIdx.x] = m.best;
+            bkey[blockIdx.x] = m.key;
+            __threadfence();
+            last = atomicAdd(done, 1) == (int)gridDim.x - 1;
+        }
+        __syncthreads();
+        if (!last) return;
+        __threadfence();  // the other blocks' results
+        m = LeastLimit();
+        for (int b = threadIdx.x; b < (int)gridDim.x; b += AT) m.take(bval[b], bkey[b]);
+        block_least(m);
+    }
+    if (threadIdx.x != 0) return;
+    *done = 0;
+    counts[slot ^ 1] = 0;
+    dt_apply(g, X, C, m, dt, LX, acc);
 }
 
 }  // namespace
@@ -464,7 +497,8 @@ struct r3d_adj_ctx {
     int nsteps = 0;
     int nf = 5;                     // primaries: 5, or 8 with LMAG
     size_t fe = 0;                  // doubles per field array
-    std::vector<double*> ckpt;      // X at steps 0, K, 2K, ...
+    std::vector<double*> ckpt;      // X at steps K, 2K, ... (at step 0: x0)
+    double* checkpoint(int s) const { return s ? ckpt[s - 1] : x0; }
     std::vector<double*> segx, seg1, seg2;  // X_n, X1, X2 of the steps of one segment
     std::vector<double> segdt;
     double* dt_pinned = nullptr;    // dt of the recomputed steps, read back once per segment
@@ -478,8 +512,10 @@ struct r3d_adj_ctx {
     double* acc = nullptr;          // g_ore, g_tk, <F, lamF>, g_theta, dt's d/dRe, g_tb
     double dJ_dtb = 0.0;            // of the last backward
     double* part = nullptr;         // k_ke block sums
-    double* bval = nullptr;
+    double* bval = nullptr;         // k_dt_adj: the blocks' least limits and their keys
     long* bkey = nullptr;
+    int* hits = nullptr;            // cells listed in either slot, blocks of k_dt_adj done
+    long* hit_cell = nullptr;
     double J = 0.0;
     double fwd_ms = 0.0, bwd_ms = 0.0;
     unsigned long long bytes = 0;
@@ -567,9 +603,14 @@ int objective(r3d_adj_ctx* a, const double* x, double* lx, double* J) {
     return R3D_OK;
 }
 
-// LO = LB + (dF/dX)^T (ca LA + cb LB) at the state x.
+DtHits dt_hits(const r3d_adj_ctx* a, double dt, int slot) {
+    return {dt / a->work->C.sff, a->hits + slot, a->hit_cell};
+}
+
+// LO = LB + (dF/dX)^T (ca LA + cb LB) at the state x.  slot >= 0: also list the
+// cells of x that may set dt.
 int vjp(r3d_adj_ctx* a, const double* x, const double* la, double ca, const double* lb, double cb,
-        double* lo) {
+        double* lo, double dt = 0.0, int slot = -1) {
     r3d_hip_ctx* w = a->work;
     const Geo& g = w->g;
     if (a->tiled) {
@@ -577,11 +618,15 @@ int vjp(r3d_adj_ctx* a, const double* x, const double* la, double ca, const doub
         const dim3 grid((p.blocks() + 7) / 8 * 8), blk(VJP_THREADS);
         auto buf = [&](const double* b) { return VjpBuf{const_cast<double*>(b), (long)a->fe}; };
         const VjpBuf bx = buf(x), ba = buf(la ? la : lb), bb = buf(lb), bo = buf(lo);
-#define R3D_VJP(MAG)                                                                            \
-    hipLaunchKernelGGL(k_vjp<MAG>, grid, blk, 0, w->stream, g, bx, w->C, w->M, ba,               \
-                       la ? ca : 0.0, bb, cb, bo, a->acc, p.ntx, p.nty, p.kq, p.krem, (int)p.blocks())
-        if (a->nf == 8) R3D_VJP(true);
-        else R3D_VJP(false);
+        const DtHits h = dt_hits(a, dt, slot < 0 ? 0 : slot);
+#define R3D_VJP(MAG, DT)                                                                         \
+    hipLaunchKernelGGL((k_vjp<MAG, DT>), grid, blk, 0, w->stream, g, bx, w->C, w->M, ba,          \
+                       la ? ca : 0.0, bb, cb, bo, a->acc, p.ntx, p.nty, p.kq, p.krem,             \
+                       (int)p.blocks(), h)
+        if (a->nf == 8 && slot >= 0) R3D_VJP(true, true);
+        else if (a->nf == 8) R3D_VJP(true, false);
+        else if (slot >= 0) R3D_VJP(false, true);
+        else R3D_VJP(false, false);
 #undef R3D_VJP
         HIPCHK(hipGetLastError());
         return R3D_OK;
@@ -609,14 +654,13 @@ int bcon_adj(r3d_adj_ctx* a, const double* x, double* lx) {
     return R3D_OK;
 }
 
-int dt_adjoint(r3d_adj_ctx* a, const double* x, double dt, double* lx) {
+// The limits' part of LX, from the cells that the transpose of stage 1 listed
+// in `slot` (none by k_flux_vjp).
+int dt_adjoint(r3d_adj_ctx* a, const double* x, double dt, int slot, double* lx) {
     r3d_hip_ctx* w = a->work;
-    const int nb = blocks_for(w->g);
-    hipLaunchKernelGGL(k_dt_argmin, dim3(nb), dim3(AT), 0, w->stream, w->g,
-                       state_of(a, (double*)x), w->C, w->M, a->bval, a->bkey);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_dt_apply, dim3(1), dim3(64), 0, w->stream, w->g, state_of(a, (double*)x),
-                       w->C, a->bval, a->bkey, nb, dt, state_of(a, lx), a->acc);
+    hipLaunchKernelGGL(k_dt_adj, dim3(blocks_for(w->g)), dim3(AT), 0, w->stream, w->g,
+                       state_of(a, (double*)x), w->C, w->M, dt_hits(a, dt, slot), a->hits, slot,
+                       a->hits + 2, a->bval, a->bkey, dt, state_of(a, lx), a->acc);
     HIPCHK(hipGetLastError());
     return R3D_OK;
 }
@@ -654,7 +698,9 @@ int r3d_adj_create(const r3d_hip_cfg* cfg, int checkpoint_every, r3d_adj_ctx** o
     if (hipMalloc((void**)&a->acc, 6 * sizeof(double)) != hipSuccess ||
         hipMalloc((void**)&a->part, ADJ_BLOCKS * sizeof(double)) != hipSuccess ||
         hipMalloc((void**)&a->bval, ADJ_BLOCKS * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&a->bkey, ADJ_BLOCKS * sizeof(long)) != hipSuccess)
+        hipMalloc((void**)&a->bkey, ADJ_BLOCKS * sizeof(long)) != hipSuccess ||
+        hipMalloc((void**)&a->hits, 3 * sizeof(int)) != hipSuccess ||
+        hipMalloc((void**)&a->hit_cell, DT_HITS * sizeof(long)) != hipSuccess)
         return fail(set_err(R3D_ENOMEM, "adjoint: small buffers"));
     for (auto* v : {&a->segx, &a->seg1, &a->seg2}) {
         v->assign(a->K, nullptr);
@@ -692,7 +738,8 @@ int r3d_adj_destroy(r3d_adj_ctx* a) {
                       a->bval, a->scratch})
         if (p) (void)hipFree(p);
     if (a->dt_pinned) (void)hipHostFree(a->dt_pinned);
-    if (a->bkey) (void)hipFree(a->bkey);
+    for (void* p : {(void*)a->bkey, (void*)a->hits, (void*)a->hit_cell})
+        if (p) (void)hipFree(p);
     if (a->seg_bufs) (void)hipFree(a->seg_bufs);
     for (auto* v : {&a->ckpt, &a->segx, &a->seg1, &a->seg2})
         for (double* p : *v)
@@ -739,7 +786,7 @@ int r3d_adj_forward(r3d_adj_ctx* a, int nsteps, double* J) {
     if (!w->metrics_set) return set_err(R3D_ESTATE, "metrics not uploaded");
     const auto t0 = std::chrono::steady_clock::now();
     const int nck = (nsteps + a->K - 1) / a->K;
-    while ((int)a->ckpt.size() < nck) {
+    while ((int)a->ckpt.size() < nck - 1) {
         double* p = nullptr;
         if ((rc = alloc_state(a, &p))) return rc;
         a->ckpt.push_back(p);
@@ -748,24 +795,26 @@ int r3d_adj_forward(r3d_adj_ctx* a, int nsteps, double* J) {
     a->nsteps = 0;
     if ((rc = seg_outer_planes(a))) return rc;
     w->cur = 0;
-    if ((rc = put_state(a, a->x0))) return rc;
+    // a run of one segment reads X0 itself and writes into the segment buffers
+    w->next_valid = false;
+    if (nck > 1 && (rc = put_state(a, a->x0))) return rc;
     r3d_hip_scalars s0{};
     if ((rc = r3d_hip_set_scalars(w, &s0))) return rc;
     const int n0 = (nck - 1) * a->K;  // first step of the last segment
     for (int n = 0; n < n0; ++n) {
-        if (n % a->K == 0 && (rc = get_state(a, a->ckpt[n / a->K]))) return rc;
+        if (n && n % a->K == 0 && (rc = get_state(a, a->checkpoint(n / a->K)))) return rc;
         if ((rc = r3d_hip_step(w, 1, 3))) return rc;
     }
     // The last segment: its checkpoint, then its steps with the stage outputs
     // redirected into the segment buffers (as the backward's recompute writes
     // them) and the final state into xfinal.  The dt of step n0 is already
     // reduced (next_valid is kept), so the steps are those of the plain path.
-    if ((rc = get_state(a, a->ckpt[nck - 1]))) return rc;
+    if (nck > 1 && (rc = get_state(a, a->checkpoint(nck - 1)))) return rc;
     {
         double* own[2][NXF];
         std::memcpy(own, w->xs, sizeof own);
         w->cur = 0;
-        for (int f = 0; f < a->nf; ++f) w->xs[0][f] = a->ckpt[nck - 1] + f * a->fe;
+        for (int f = 0; f < a->nf; ++f) w->xs[0][f] = a->checkpoint(nck - 1) + f * a->fe;
         for (int n = n0; n < nsteps; ++n) {
             double* outs[3] = {a->seg1[n - n0], a->seg2[n - n0],
                                n + 1 < nsteps ? a->segx[n + 1 - n0] : a->xfinal};
@@ -806,6 +855,7 @@ int backward(r3d_adj_ctx* a, double* const* grad, double* dJ_dre, double* dJ_dth
     HIPCHK(hipMemsetAsync(L, 0, a->fe * a->nf * sizeof(double), w->stream));
     if ((rc = objective(a, a->xfinal, L, &Jdummy))) return rc;  // L = dJ/dX_N (B: 0)
     HIPCHK(hipMemsetAsync(a->acc, 0, 6 * sizeof(double), w->stream));
+    HIPCHK(hipMemsetAsync(a->hits, 0, 3 * sizeof(int), w->stream));
     const double g1 = C.gam[0], g2 = C.gam[1], g3 = C.gam[2];
     const double z1 = C.zeta[0], z2 = C.zeta[1];
     const int N = a->nsteps, nseg = (N + a->K - 1) / a->K;
@@ -822,7 +872,7 @@ int backward(r3d_adj_ctx* a, double* const* grad, double* dJ_dre, double* dJ_dth
             double* own[2][NXF];
             std::memcpy(own, w->xs, sizeof own);
             w->cur = 0;
-            for (int f = 0; f < a->nf; ++f) w->xs[0][f] = a->ckpt[sgm] + f * a->fe;
+            for (int f = 0; f < a->nf; ++f) w->xs[0][f] = a->checkpoint(sgm) + f * a->fe;
             w->next_valid = false;
             for (int n = n0; n < n1; ++n) {
                 // the last step's X_{n+1} (a checkpoint or the final state) is
@@ -843,13 +893,12 @@ int backward(r3d_adj_ctx* a, double* const* grad, double* dJ_dre, double* dJ_dth
             for (int n = n0; n < n1; ++n) a->segdt[n - n0] = a->dt_pinned[n - n0];
         }
         for (int n = n1 - 1; n >= n0; --n) {
-            const double* xn = n == n0 ? a->ckpt[sgm] : a->segx[n - n0];
+            const double* xn = n == n0 ? a->checkpoint(sgm) : a->segx[n - n0];
             const double* x1b = a->seg1[n - n0];
             const double* x2b = a->seg2[n - n0];
             const double* xn1 =
-                n + 1 < n1 ? a->segx[n + 1 - n0] : (n1 == N ? a->xfinal : a->ckpt[sgm + 1]);
+                n + 1 < n1 ? a->segx[n + 1 - n0] : (n1 == N ? a->xfinal : a->checkpoint(sgm + 1));
             const double dt = a->segdt[n - n0];
-            HIPCHK(hipMemsetAsync(a->acc + 2, 0, sizeof(double), w->stream));
             // stage 3: L = lam X_{n+1} -> B^T; lamF = g3 dt L; lamZ2 = L
             if ((rc = bcon_adj(a, xn1, L))) return rc;
             if ((rc = vjp(a, x2b, nullptr, 0.0, L, g3 * dt, Mb))) return rc;
@@ -858,8 +907,9 @@ int backward(r3d_adj_ctx* a, double* const* grad, double* dJ_dre, double* dJ_dth
             if ((rc = vjp(a, x1b, L, z2 * dt, Mb, g2 * dt, Nb))) return rc;
             // stage 1: lamF = z1 dt lamZ1 + g1 dt lamX1; Z0 = X_n
             if ((rc = bcon_adj(a, x1b, Nb))) return rc;
-            if ((rc = vjp(a, xn, Mb, z1 * dt, Nb, g1 * dt, L))) return rc;
-            if (C.dtfix <= 0.0 && (rc = dt_adjoint(a, xn, dt, L))) return rc;
+            const int slot = C.dtfix > 0.0 ? -1 : n & 1;
+            if ((rc = vjp(a, xn, Mb, z1 * dt, Nb, g1 * dt, L, dt, slot))) return rc;
+            if (slot >= 0 && (rc = dt_adjoint(a, xn, dt, slot, L))) return rc;
         }
     }
     double acc[6];

@@ -94,6 +94,9 @@ struct VjpLds {
     double zm[4][VJP_KC + 2];  // dzz, d2zz, rkapa, dkapa of planes k0-1 .. k1+1
     double xm[3][VW + 2], ym[3][VH + 2];  // hx dxx, lx1, lx2 of the columns; the rows'
     double red[8][3];
+    // DT: ddx of the columns, ddy of the rows, ddz of the planes; the bounds'
+    // constants (a lane that held them across the z loop would spill)
+    double xd[VW + 2], yd[VH + 2], zd[VJP_KC + 2], scr[5];
     double s[MAG ? 7 : 4][VH + 4][VW + 4];
     double e[MAG ? (int)NVE_MAG : (int)NVE][VH + 2][VW + 2];
     // MAG: the sums of plane p - 1 wait here while plane p's emissions are
@@ -163,12 +166,24 @@ __device__ __forceinline__ Raw vjp_load(const VjpBuf& x, long pp, int k, uint32_
     return r;
 }
 
-template <bool MAG>
+// The cells of X that may hold the least time-step limit (lim, known from the
+// forward run): those that fail the division-free bounds of dt_screen.  Their
+// indices, up to DT_HITS of them, and how many there are.
+constexpr int DT_HITS = 1024;
+struct DtHits {
+    double lim;
+    int* count;
+    long* cell;
+};
+
+// DT: also list the cells of X that may set the step's dt (the transpose of a
+// step's first stage reads the state that dt was taken from).
+template <bool MAG, bool DT>
 __global__ __launch_bounds__(VJP_THREADS) void k_vjp(const Geo g, const VjpBuf X, const Consts C,
                                                      const Metrics M, const VjpBuf LA, double ca,
                                                      const VjpBuf LB, double cb, const VjpBuf LO,
                                                      double* acc, int ntx, int nty, int kq,
-                                                     int krem, int nblocks) {
+                                                     int krem, int nblocks, const DtHits H) {
     constexpr int NF = MAG ? 8 : 5;
     __shared__ VjpLds<MAG> L;
     const int t = logical_block();
@@ -215,6 +230,7 @@ __global__ __launch_bounds__(VJP_THREADS) void k_vjp(const Geo g, const VjpBuf X
 
     for (int q = threadIdx.x; q < 4 * (VJP_KC + 2); q += VJP_THREADS) {
         const int f = q / (VJP_KC + 2), kk = k0 - 1 + q % (VJP_KC + 2);
+        if (DT && f == 0 && kk >= k0 && kk <= k1) L.zd[kk - k0 + 1] = M.ddz[kk];
         if (kk <= k1 + 1) {
             const double* src = f == 0 ? M.dzz : f == 1 ? M.d2zz : f == 2 ? M.rkapa : M.dkapa;
             L.zm[f][kk - k0 + 1] = src[kk];
@@ -226,15 +242,26 @@ __global__ __launch_bounds__(VJP_THREADS) void k_vjp(const Geo g, const VjpBuf X
     for (int q = threadIdx.x; q < VW + 2 + VH + 2; q += VJP_THREADS) {
         if (q < VW + 2) {
             const int i = wrap(i0 + q - 1, g.npx);
+            if (DT) L.xd[q] = M.ddx[i];
             L.xm[0][q] = C.hx * M.dxx[i];
             L.xm[1][q] = C.hx * M.d2xx[i];
             L.xm[2][q] = l2(C.h2x, M.dxx[i]);
         } else {
             const int j = wrap(j0 + q - (VW + 2) - 1, g.npy);
+            if (DT) L.yd[q - (VW + 2)] = M.ddy[j];
             L.ym[0][q - (VW + 2)] = C.hy * M.dyy[j];
             L.ym[1][q - (VW + 2)] = C.hy * M.d2yy[j];
             L.ym[2][q - (VW + 2)] = l2(C.h2y, M.dyy[j]);
         }
+    }
+
+    if (DT && threadIdx.x == 0) {
+        const double t = H.lim * (1.0 + 1e-9);  // far above the rounding of limits and bounds
+        L.scr[0] = t;
+        L.scr[1] = t * t;
+        L.scr[2] = 0.5 * C.repr * C.cv;
+        L.scr[3] = 0.375 * C.re;
+        L.scr[4] = 0.5 * C.rm;
     }
 
     Raw r2n{};  // the second cell's momenta, density and field on the next plane
@@ -547,6 +574,24 @@ __global__ __launch_bounds__(VJP_THREADS) void k_vjp(const Geo g, const VjpBuf X
                        LW * C.grav * sc.ro;
                 gtk += LT * R * cond;
                 gore += LT * R * C.ocv * (q1 + C.c43 * q3);
+                if constexpr (DT) {
+                    const double dd = dmin(dmin(L.xd[c], L.yd[r]), L.zd[pl]);
+                    const double d2 = dd * dd, x = d2 * sc.ro, t = L.scr[0];
+                    double gg = C.gamma * sc.tt;
+                    if constexpr (MAG)
+                        gg += (sc.bx * sc.bx + sc.by * sc.by + sc.bz * sc.bz) * C.obeta * R;
+                    const double uu = sc.u * sc.u + sc.v * sc.v + sc.w * sc.w;
+                    bool hit = !(sc.ro > 0.0 && sc.tt > 0.0 && rk > 0.0);
+                    hit |= !(x * L.scr[2] > t * rk);
+                    hit |= !(x * L.scr[3] > t);
+                    hit |= !(d2 > L.scr[1] * (5.0 * uu + 1.25 * gg));
+                    if constexpr (MAG) hit |= !(d2 * L.scr[4] > t);
+                    if (hit && out) {
+                        const int n = atomicAdd(H.count, 1);
+                        if (n < DT_HITS)
+                            H.cell[n] = ((long)(p - 1) * g.npy + (gj - 1)) * g.npx + (gi - 1);
+                    }
+                }
                 if (C.lrot) {
                     const double xu = -LV * C.omz, xv = LU * C.omz - LW * C.omx, xw = LV * C.omx;
                     a.ru += xu;
