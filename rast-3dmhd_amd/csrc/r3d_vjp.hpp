@@ -40,17 +40,21 @@ namespace r3d {
 // cells reach one cell further, so the lanes of wave 6 also publish the state
 // of the row beyond theirs, and 24 more lanes of wave 7 the columns beyond.
 // Per plane p: publish the state, barrier, form the emitted quantities and
-// publish them, barrier, collect.  What plane p emits in z stays in the
-// column's registers: plane p - 1 is finished with it and stored, and plane
-// p + 1 starts from it.
+// publish them, barrier, collect.  Without MAG two planes of each fit into LDS:
+// the state is published a plane ahead, and one barrier a plane is left (between
+// it and the next, a wave writes the planes that no slower one still reads).
+// What plane p emits in z stays in the column's registers: plane p - 1 is
+// finished with it and stored, and plane p + 1 starts from it.
 //
-// At 128x128x256 a launch takes 219 us (MHD 414), where the bytes it cannot do
-// without (the state, LA, LB and LO once each: 160 and 256 a cell) take 143 (229)
-// at the copy rate of the card.  The two barriers a plane with two waves per
-// SIMD, and the arithmetic (some 420 and 660 FP64 instructions a wave and plane)
-// bound it.  A kernel that added every cell's 19-point entries into an LDS ring
-// with LDS atomics, and its frame with global ones into a zeroed LO, took 812
-// us (MHD 1581) and 22 (32) for the zeroing.
+// At 128x128x256 a launch takes 217 us (MHD 382; 230 and 441 where it also lists
+// the cells that may set dt), where the bytes it cannot do without (the state,
+// LA, LB and LO once each: 160 and 256 a cell) take 143 (229) at the copy rate of
+// the card; with two barriers a plane hydro took 226 (248).  Two waves per SIMD,
+// six of eight collecting, and the arithmetic (some 420 and 660 FP64 instructions
+// a wave and plane) bound it: of the wave cycles 42% (MHD 52%) wait for memory or
+// a barrier, 29% (22%) to issue.  A kernel that added every cell's 19-point
+// entries into an LDS ring with LDS atomics, and its frame with global ones into
+// a zeroed LO, took 812 us (MHD 1581) and 22 (32) for the zeroing.
 constexpr int VW = 32, VH = 12, VJP_THREADS = 512;
 constexpr int VJP_KC = 128;  // planes of a chunk at most
 
@@ -97,8 +101,9 @@ struct VjpLds {
     // DT: ddx of the columns, ddy of the rows, ddz of the planes; the bounds'
     // constants (a lane that held them across the z loop would spill)
     double xd[VW + 2], yd[VH + 2], zd[VJP_KC + 2], scr[5];
-    double s[MAG ? 7 : 4][VH + 4][VW + 4];
-    double e[MAG ? (int)NVE_MAG : (int)NVE][VH + 2][VW + 2];
+    static constexpr int NB = MAG ? 1 : 2;  // planes held of each
+    double s[NB][MAG ? 7 : 4][VH + 4][VW + 4];
+    double e[NB][MAG ? (int)NVE_MAG : (int)NVE][VH + 2][VW + 2];
     // MAG: the sums of plane p - 1 wait here while plane p's emissions are
     // formed (in registers they would spill)
     double park[MAG ? 11 : 1][MAG ? 6 * 64 : 1];
@@ -149,6 +154,36 @@ struct VjpBuf {
     long fe;
     __device__ __forceinline__ double* operator[](int f) const { return p + f * fe; }
 };
+
+// The state x into a plane of L.s, at the lane's cell (p0) and its second one
+// (p2).  A macro: as a lambda it changes the register allocation of the MAG
+// kernel, for 416 us a launch instead of 382.
+#define R3D_VJP_PUBLISH(p0, p2, x)                      \
+    do {                                                \
+        if (!FLUX && second_) {                         \
+            const Raw q = r2n;                          \
+            const double ri = 1.0 / q.ro;               \
+            p2[VS_U * VSP + VSR + 1] = q.ru * ri;       \
+            p2[VS_V * VSP + VSR + 1] = q.rv * ri;       \
+            p2[VS_W * VSP + VSR + 1] = q.rw * ri;       \
+            if constexpr (MAG) {                        \
+                p2[VS_BX * VSP + VSR + 1] = q.bx;       \
+                p2[VS_BY * VSP + VSR + 1] = q.by;       \
+                p2[VS_BZ * VSP + VSR + 1] = q.bz;       \
+            }                                           \
+        }                                               \
+        if (FLUX || emits) {                            \
+            p0[VS_U * VSP + VSR + 1] = x.u;             \
+            p0[VS_V * VSP + VSR + 1] = x.v;             \
+            p0[VS_W * VSP + VSR + 1] = x.w;             \
+            p0[VS_T * VSP + VSR + 1] = x.tt;            \
+            if constexpr (MAG) {                        \
+                p0[VS_BX * VSP + VSR + 1] = x.bx;       \
+                p0[VS_BY * VSP + VSR + 1] = x.by;       \
+                p0[VS_BZ * VSP + VSR + 1] = x.bz;       \
+            }                                           \
+        }                                               \
+    } while (0)
 
 template <bool MAG>
 __device__ __forceinline__ Raw vjp_load(const VjpBuf& x, long pp, int k, uint32_t voff) {
@@ -333,23 +368,31 @@ __global__ __launch_bounds__(VJP_THREADS) void k_vjp(const Geo g, const VjpBuf X
     // barriers over the same planes.
     const bool second_ = second;
     // (the bases are those of the cell's lower left neighbour)
-    ldouble* sb = lds_of(&L.s[0][0][0]) + r * VSR + c;
-    ldouble* sb2 = lds_of(&L.s[0][0][0]) + r2 * VSR + c2;
-    ldouble* eb = lds_of(&L.e[0][0][0]) + (r - 1) * VER + (c - 1);
+    ldouble* sb = lds_of(&L.s[0][0][0][0]) + r * VSR + c;
+    ldouble* sb2 = lds_of(&L.s[0][0][0][0]) + r2 * VSR + c2;
+    ldouble* eb = lds_of(&L.e[0][0][0][0]) + (r - 1) * VER + (c - 1);
     ldouble* eb2 = eb + NVE * VEP;
     ldouble* pb = lds_of(&L.park[0][0]) + threadIdx.x;
     auto zloop = [&](auto flux_c) {
     constexpr bool FLUX = decltype(flux_c)::value;
+    constexpr int SBUF = MAG ? 0 : 4 * VSP, EBUF = MAG ? 0 : NVE * VEP;
     if (!FLUX && second_) fetch2(k0 - 1);
+    if constexpr (!MAG) {  // the first plane; the loop publishes a plane ahead
+        const int par = (k0 - 1) & 1;
+        ldouble *const s0 = sb + par * SBUF, *const s2 = sb2 + par * SBUF;
+        R3D_VJP_PUBLISH(s0, s2, sc);
+        if (!FLUX && second_) fetch2(k0);
+    }
     // The next plane's lamF and the state after it (none past the last): issued
     // with the whole plane ahead of their use where the registers allow it, with
     // MAG only once the emissions are formed (earlier spills: 488 against 414 us
-    // a launch at 128x128x256; without MAG late issue takes 269 against 218 us).
+    // a launch at 128x128x256 when measured; without MAG late issue took 269
+    // against 218 us).
     auto fetch_next = [&](int p) {
         if (p == k1 + 1) return;
         rn = vjp_load<MAG>(X, g.pp, min(p + 2, g.npz + 1), voff);
         if (p + 1 <= g.npz) fetch_lam(p + 1);
-        if (!FLUX && second_) fetch2(p + 1);
+        if (!FLUX && second_) fetch2(MAG ? p + 1 : min(p + 2, g.npz + 1));
     };
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();  // the metrics are in LDS
@@ -382,32 +425,18 @@ __global__ __launch_bounds__(VJP_THREADS) void k_vjp(const Geo g, const VjpBuf X
             zpart(a, sc, Q, -h, z2 + z1, lcb, outer ? 0.0 : (wall ? 4.0 : 1.0),
                   L.zm[2][pl - 1], L.zm[3][pl - 1]);
         }
-        if (!FLUX && second_) {
-            const Raw q = r2n;
-            const double ri = 1.0 / q.ro;
-            sb2[VS_U * VSP + VSR + 1] = q.ru * ri;
-            sb2[VS_V * VSP + VSR + 1] = q.rv * ri;
-            sb2[VS_W * VSP + VSR + 1] = q.rw * ri;
-            if constexpr (MAG) {
-                sb2[VS_BX * VSP + VSR + 1] = q.bx;
-                sb2[VS_BY * VSP + VSR + 1] = q.by;
-                sb2[VS_BZ * VSP + VSR + 1] = q.bz;
-            }
-        }
-        if (FLUX || emits) {
-            sb[VS_U * VSP + VSR + 1] = sc.u;
-            sb[VS_V * VSP + VSR + 1] = sc.v;
-            sb[VS_W * VSP + VSR + 1] = sc.w;
-            sb[VS_T * VSP + VSR + 1] = sc.tt;
-            if constexpr (MAG) {
-                sb[VS_BX * VSP + VSR + 1] = sc.bx;
-                sb[VS_BY * VSP + VSR + 1] = sc.by;
-                sb[VS_BZ * VSP + VSR + 1] = sc.bz;
-            }
-        }
+        ldouble *sbc = sb, *ebc = eb;  // this plane's
+        if constexpr (MAG) R3D_VJP_PUBLISH(sb, sb2, sc);
         const VjpCol sp = vjp_derive<MAG>(rn);
-        if constexpr (!MAG) fetch_next(p);
-        __syncthreads();
+        if constexpr (!MAG) {
+            const int par = p & 1;
+            sbc = sb + par * SBUF;
+            ebc = eb + par * EBUF;
+            ldouble *const s0 = sb + (par ^ 1) * SBUF, *const s2 = sb2 + (par ^ 1) * SBUF;
+            R3D_VJP_PUBLISH(s0, s2, sp);
+            fetch_next(p);
+        }
+        if constexpr (MAG) __syncthreads();
 
         VjpUp q{};  // what this plane emits in z
         const double hz0 = C.hz * L.zm[0][pl], lz1 = C.hz * L.zm[1][pl];
@@ -418,8 +447,8 @@ __global__ __launch_bounds__(VJP_THREADS) void k_vjp(const Geo g, const VjpBuf X
             const double R = sc.ri;
             const double hx0 = L.xm[0][c], hy0 = L.ym[0][r];
 #define E_(f, dr, dc) \
-    ((f) < NVE ? eb : eb2)[((f) - ((f) < NVE ? 0 : (int)NVE)) * VEP + (1 + (dr)) * VER + 1 + (dc)]
-#define S_(f, dr, dc) sb[(f) * VSP + (1 + (dr)) * VSR + 1 + (dc)]
+    ((f) < NVE ? ebc : eb2)[((f) - ((f) < NVE ? 0 : (int)NVE)) * VEP + (1 + (dr)) * VER + 1 + (dc)]
+#define S_(f, dr, dc) sbc[(f) * VSP + (1 + (dr)) * VSR + 1 + (dc)]
 #define DXS(f) ((S_(f, 0, 1) - S_(f, 0, -1)) * hx0)
 #define DYS(f) ((S_(f, 1, 0) - S_(f, -1, 0)) * hy0)
             const double ux = DXS(VS_U), vx = DXS(VS_V), wx = DXS(VS_W);
