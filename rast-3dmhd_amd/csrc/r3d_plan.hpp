@@ -1,5 +1,6 @@
-// r3d_plan.hpp - how a run's stage kernel is cut into workgroups: tile rows
-// and z chunks (host only; the CPU tests run it directly).
+// r3d_plan.hpp - how a run's stage kernel and the adjoint's flux transpose are
+// cut into workgroups: tile rows and z chunks (host only; the CPU tests run it
+// directly).
 #pragma once
 
 #include <initializer_list>
@@ -134,6 +135,37 @@ inline StagePlan plan_stage(int npx, int npy, int npz, bool lmag, bool feature, 
                 best = p;
             }
         }
+    }
+    return best;
+}
+
+// The adjoint's flux transpose (r3d_vjp.hpp): tiles of VH rows x VW columns, each
+// marching up a chunk of at most VJP_KC planes.
+constexpr int VW = 32, VH = 12, VJP_KC = 128;
+
+// ntx x nty tiles, nkc chunks of kq planes, the first krem one more.
+struct VjpPlan {
+    int ntx, nty, nkc, kq, krem;
+    long blocks() const { return (long)ntx * nty * nkc; }
+};
+// One workgroup fills a CU, so a launch runs in rounds of one tile per CU; a
+// chunk costs its planes and some four more (the plane on either side, whose
+// emissions it forms too, and the filling of the first ones).  The cheapest
+// number of equal chunks by that.
+inline VjpPlan plan_vjp(int npx, int npy, int npz, int cus) {
+    VjpPlan p{(npx + VW - 1) / VW, (npy + VH - 1) / VH, 0, 0, 0}, best{};
+    double least = 1e300;
+    for (int nkc = (npz + VJP_KC - 1) / VJP_KC; nkc <= npz; ++nkc) {
+        p.nkc = nkc;
+        p.kq = npz / nkc;
+        p.krem = npz % nkc;
+        const long rounds = (p.blocks() + cus - 1) / cus;
+        const double t = (double)rounds * (p.kq + (p.krem > 0) + 4.0);
+        if (t < least) {
+            least = t;
+            best = p;
+        }
+        if (rounds > 16) break;  // only the filling grows
     }
     return best;
 }

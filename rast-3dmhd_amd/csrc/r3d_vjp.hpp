@@ -25,11 +25,14 @@
 // <F, lamF> and its derivatives by ore and tk come from the same sums: what is
 // linear in a difference is paired with its transpose (sum F.lam = sum
 // m_c u DX(L_c) + P a(P) + u a_visc(u) + ...), the rest is evaluated at the cell.
-// For that the two outer planes count as receivers too, of these sums alone.
+// For that the two outer planes count as receivers too, of these sums alone, in
+// the chunks that own the wall planes (a chunk from plane 2 passes over plane 1
+// as well, for its emissions).
 #pragma once
 
 #include "r3d_adj.hpp"
 #include "r3d_ctx.hpp"
+#include "r3d_plan.hpp"
 
 namespace r3d {
 
@@ -55,35 +58,7 @@ namespace r3d {
 // a barrier, 29% (22%) to issue.  A kernel that added every cell's 19-point
 // entries into an LDS ring with LDS atomics, and its frame with global ones into
 // a zeroed LO, took 812 us (MHD 1581) and 22 (32) for the zeroing.
-constexpr int VW = 32, VH = 12, VJP_THREADS = 512;
-constexpr int VJP_KC = 128;  // planes of a chunk at most
-
-// ntx x nty tiles, nkc chunks of kq planes, the first krem one more.
-struct VjpPlan {
-    int ntx, nty, nkc, kq, krem;
-    long blocks() const { return (long)ntx * nty * nkc; }
-};
-// One workgroup fills a CU, so a launch runs in rounds of one tile per CU; a
-// chunk costs its planes and some four more (the plane on either side, whose
-// emissions it forms too, and the filling of the first ones).  The cheapest
-// number of equal chunks by that.
-inline VjpPlan plan_vjp(int npx, int npy, int npz, int cus) {
-    VjpPlan p{(npx + VW - 1) / VW, (npy + VH - 1) / VH, 0, 0, 0}, best{};
-    double least = 1e300;
-    for (int nkc = (npz + VJP_KC - 1) / VJP_KC; nkc <= npz; ++nkc) {
-        p.nkc = nkc;
-        p.kq = npz / nkc;
-        p.krem = npz % nkc;
-        const long rounds = (p.blocks() + cus - 1) / cus;
-        const double t = (double)rounds * (p.kq + (p.krem > 0) + 4.0);
-        if (t < least) {
-            least = t;
-            best = p;
-        }
-        if (rounds > 16) break;  // only the filling grows
-    }
-    return best;
-}
+constexpr int VJP_THREADS = 512;
 
 // LDS arrays: the state at rows -1..VH+2, columns -1..VW+2
 enum { VS_U = 0, VS_V, VS_W, VS_T, VS_BX, VS_BY, VS_BZ };
@@ -658,8 +633,9 @@ __global__ __launch_bounds__(VJP_THREADS) void k_vjp(const Geo g, const VjpBuf X
             }
             const int k = p - 1;
             const bool done = k >= k0 && k <= k1;
-            if (emit && (done || k == 0)) {
-                const bool wall = p == g.npz, outer = k == 0;
+            const bool outer = k == 0 && k0 == 1;
+            if (emit && (done || outer)) {
+                const bool wall = p == g.npz;
                 const bool one = (wall && C.mag_bot) || outer;
                 zpart(A, sm, q, hz0, lz2 - lz1,
                       one ? (outer ? 0.0 : -4.0 * lz1 - 5.0 * lz2) : lz2 - lz1,
