@@ -757,16 +757,18 @@ int r3d_adj_set_metrics(r3d_adj_ctx* a, const r3d_hip_metrics* m) {
 namespace {
 int set_initial(r3d_adj_ctx* a, const double* const* fields, bool device) {
     if (!a || !fields) return set_err(R3D_EINVAL, "null argument");
-    for (int f = 0; f < a->nf; ++f) {
+    // a refused call leaves X0, which the backward starts its first segment from
+    for (int f = 0; f < a->nf; ++f)
         if (!fields[f]) return set_err(R3D_EINVAL, "field %d missing", f);
+    a->nsteps = 0;
+    a->seg_outer = false;
+    a->kept_last = false;
+    for (int f = 0; f < a->nf; ++f) {
         double* src = const_cast<double*>(fields[f]);
         int rc = device ? global_copy_device(a->work, a->x0 + f * a->fe, src, false)
                         : global_copy(a->work, a->x0 + f * a->fe, src, false);
         if (rc) return rc;
     }
-    a->nsteps = 0;
-    a->seg_outer = false;
-    a->kept_last = false;
     return R3D_OK;
 }
 }  // namespace
