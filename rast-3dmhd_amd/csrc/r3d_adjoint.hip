@@ -398,9 +398,14 @@ __device__ __forceinline__ void block_least(LeastLimit& m) {
 // One thread: LX[cell] += sff * lam_dt * dL/dX at the cell and limit of the
 // minimum, lam_dt = acc[2] / dt, and acc[4] += sff * lam_dt * dL/dRe; acc[2]
 // is spent.  At a cell at rest the advective limit's velocity derivative is
-// taken as 0.
+// taken as 0.  No cell sets dt where every limit is no number (a run that blew
+// up): there is nothing to add then.
 __device__ void dt_apply(const Geo& g, const State& X, const Consts& C, const LeastLimit& m,
                          double dt, const State& LX, double* acc) {
+    if (m.key == LONG_MAX) {
+        acc[2] = 0.0;
+        return;
+    }
     const long q = (m.key - 1) / 4;
     const int t = (int)((m.key - 1) % 4);  // 0 advective, 1 thermal, 2 viscous
     int i, j, k;
