@@ -16,7 +16,7 @@
 // and through the thermal and viscous dt limits; theta through the boundary
 // heat-flux conditions.
 //
-// This file is compiled with -ffp-contract=fast (the transposes need no
+// This file is compiled with contraction (the transposes need no
 // reference rounding); the objective and the dt argmin, which must round as
 // the forward does, switch contraction off.
 //

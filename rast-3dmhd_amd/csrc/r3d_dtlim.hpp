@@ -24,24 +24,32 @@ __host__ __device__ __forceinline__ double dmin(double a, double b) { return b <
 // dd/sqrt(fast speed), the thermal and the viscous limit, pm[4] = min of the
 // resistive limit (MHD).  With MAG the fast speed includes the Alfven term
 // b2 = (bx^2+by^2+bz^2)*obeta/ro (src/step.cpp:144-156).
-template <bool MAG>
-__host__ __device__ __forceinline__ void dt_terms(const Consts& C, double ru, double rv, double rw,
-                                         double ro, double tt, double bx, double by, double bz,
-                                         double dd, double rk, double pm[NPART]) {
-    const double uu = (ru * ru + rv * rv + rw * rw) * (1.0 / ro) * (1.0 / ro);
-    pm[0] = dmax(pm[0], C.og * uu / tt);
-    double fast;
-    if constexpr (MAG) {
-        const double b2 = (bx * bx + by * by + bz * bz) * C.obeta / ro;
-        fast = uu + C.gamma * tt + b2 + 2.0 * sqrt(uu * (C.gamma * tt + b2));
-    } else {
-        fast = uu + C.gamma * tt + 2.0 * sqrt(uu * C.gamma * tt);
+// dt_terms rounds as the build it is compiled in (in the FMA-contracted one,
+// contracted); dt_terms_sep rounds every product and sum by itself in all of
+// them, like the exact pass over a state (k_dt).
+#define R3D_DT_TERMS(NAME, PRAGMA)                                                               \
+    template <bool MAG>                                                                          \
+    __host__ __device__ __forceinline__ void NAME(                                               \
+        const Consts& C, double ru, double rv, double rw, double ro, double tt, double bx,       \
+        double by, double bz, double dd, double rk, double pm[NPART]) {                          \
+        PRAGMA                                                                                   \
+        const double uu = (ru * ru + rv * rv + rw * rw) * (1.0 / ro) * (1.0 / ro);               \
+        pm[0] = dmax(pm[0], C.og * uu / tt);                                                     \
+        double fast;                                                                             \
+        if constexpr (MAG) {                                                                     \
+            const double b2 = (bx * bx + by * by + bz * bz) * C.obeta / ro;                      \
+            fast = uu + C.gamma * tt + b2 + 2.0 * sqrt(uu * (C.gamma * tt + b2));                \
+        } else {                                                                                 \
+            fast = uu + C.gamma * tt + 2.0 * sqrt(uu * C.gamma * tt);                            \
+        }                                                                                        \
+        pm[1] = dmin(pm[1], dd / sqrt(fast));                                                    \
+        pm[2] = dmin(pm[2], 0.5 * dd * dd * C.repr * C.cv * ro / rk);                            \
+        pm[3] = dmin(pm[3], 0.375 * dd * dd * C.re * ro);                                        \
+        if constexpr (MAG) pm[4] = dmin(pm[4], 0.5 * dd * dd * C.rm);                            \
     }
-    pm[1] = dmin(pm[1], dd / sqrt(fast));
-    pm[2] = dmin(pm[2], 0.5 * dd * dd * C.repr * C.cv * ro / rk);
-    pm[3] = dmin(pm[3], 0.375 * dd * dd * C.re * ro);
-    if constexpr (MAG) pm[4] = dmin(pm[4], 0.5 * dd * dd * C.rm);
-}
+R3D_DT_TERMS(dt_terms, )
+R3D_DT_TERMS(dt_terms_sep, _Pragma("clang fp contract(off)"))
+#undef R3D_DT_TERMS
 
 // Constants of the time-step screen, formed once per block from the
 // previous extrema: the thresholds thr_um (ogamma*UU/T) and thr_lim (every

@@ -1,11 +1,12 @@
 // r3d_fma.hip - the FMA-contracted variant of the stage kernel.
 //
 // The same source as the bit-exact stage kernel (r3d_stage.hpp), compiled in
-// this translation unit with -ffp-contract=fast and in namespace r3d_fma, so
-// that products feeding sums become fused multiply-adds.  Results differ from
-// the reference's rounding; the error against the bit-exact variant is
-// measured by tests/test_gpu_fma.py.  Boundary, dt and bookkeeping kernels
-// are shared with the bit-exact build.
+// this translation unit with -ffp-contract=fast-honor-pragmas and in namespace
+// r3d_fma, so that products feeding sums become fused multiply-adds.  Results
+// differ from the reference's rounding; the error against the bit-exact variant
+// is measured by tests/test_gpu_fma.py.  The wall cells (the boundary conditions,
+// their RK mix and their time-step limits) are not contracted, and the dt and
+// bookkeeping kernels are shared with the bit-exact build.
 #include <hip/hip_runtime.h>
 
 #define R3D_KNS r3d_fma

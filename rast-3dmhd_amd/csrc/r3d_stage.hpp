@@ -41,7 +41,7 @@
 
 // The kernels live in namespace R3D_KNS: r3d for the bit-exact build; the
 // FMA-contracted variant compiles this same code a second time, in its own
-// namespace and translation unit, with -ffp-contract=fast (r3d_fma.hip).
+// namespace and translation unit, with contraction (r3d_fma.hip).
 #ifndef R3D_KNS
 #define R3D_KNS r3d
 #endif
@@ -992,7 +992,7 @@ __device__ __forceinline__ void stage_walls(const StageArgs& a, const Consts& C,
             double b[3] = {0.0, 0.0, 0.0};
             if constexpr (MAG)
                 for (int q = 0; q < 3; ++q) b[q] = y[QBX + q];
-            dt_terms<MAG>(C, w.ru, w.rv, 0.0, ro, w.tt, b[0], b[1], b[2], met[0], met[1], pm);
+            dt_terms_sep<MAG>(C, w.ru, w.rv, 0.0, ro, w.tt, b[0], b[1], b[2], met[0], met[1], pm);
         }
     }
 }
