@@ -83,6 +83,8 @@ __device__ __forceinline__ void reduce_partials(const double* partial, int npart
     __syncthreads();
     if (threadIdx.x != 0) return;
     for (int q = 0; q < NPART; ++q) o[q] = red[0][q];
+    // not unrolled: the 80 values of 16 waves read at once would spill
+#pragma unroll 1
     for (int w = 1; w < NT / 64; ++w) {
         o[0] = dmax(o[0], red[w][0]);
         for (int q = 1; q < NPART; ++q) o[q] = dmin(o[q], red[w][q]);
