@@ -34,6 +34,16 @@ struct EnsMember {
     Metrics M;
 };
 
+// A place in the member table, which no kernel writes: through the constant
+// address space, where a kernel's own arguments lie too, its values are scalar
+// loads that no store of a stage's z loop can alias, so they are held or loaded
+// again as the registers allow.  64 members, a step: 5.07 ms (persistent launch
+// 5.19; MHD, 24 members: 3.50 and 3.62).  By-value copies of the scalars, which
+// the stores cannot alias either, fill the scalar registers and then spill: 5.12
+// (16.9; 3.65 and 11.4).
+typedef const __attribute__((address_space(4))) EnsMember* EnsTable;
+__device__ __forceinline__ const EnsMember& member(EnsTable m) { return *(const EnsMember*)m; }
+
 constexpr int ENS_DT_BLOCKS = 64;  // blocks per member of the standalone dt pass
 
 __device__ __forceinline__ StageArgs member_args(const EnsMember& e, int cur, int stage,
@@ -61,30 +71,29 @@ __device__ __forceinline__ StageArgs member_args(const EnsMember& e, int cur, in
 // One tile of one stage of member e, then its wall cells (member data read by a
 // second route there, as in k_stage), then its dt partial.
 template <int TY, int STAGE, bool MAG, int TW>
-__device__ __forceinline__ void member_tile(const EnsMember& e, int t, int cur,
+__device__ __forceinline__ void member_tile(EnsTable m, int t, int cur,
                                             StageLds<TY, STAGE, MAG, false, false, TW>& lds) {
     constexpr int ZMODE = STAGE < 2 ? 0 : 2;
     double pm[NPART];
     TileCell<TY, TW> me;
-    // copies: read through the table the constants would be loaded again after
-    // every store of the z loop, which might alias it
+    const EnsMember& e = member(m);
     const StageArgs a = member_args(e, cur, STAGE, ZMODE, STAGE == 2);
-    const Consts C = e.C;
-    const Metrics M = e.M;
-    if (stage_tile<TY, STAGE, ZMODE, MAG, false, false, TW>(a, C, M, t, lds, pm, me)) {
-        const EnsMember* w = &e;
-        asm volatile("" : "+s"(w));
-        stage_walls<TY, STAGE, ZMODE, MAG, TW>(member_args(*w, cur, STAGE, ZMODE, STAGE == 2),
-                                               w->C, w->M, me, pm);
+    if (stage_tile<TY, STAGE, ZMODE, MAG, false, false, TW>(a, e.C, e.M, t, lds, pm, me)) {
+        asm volatile("" : "+s"(m));
+        const EnsMember& w = member(m);
+        stage_walls<TY, STAGE, ZMODE, MAG, TW>(member_args(w, cur, STAGE, ZMODE, STAGE == 2), w.C,
+                                               w.M, me, pm);
     }
     if (STAGE == 2) block_partials<TileShape<TY, TW>::NW>(pm, lds.red, a.partial, t);
 }
 
 // One stage of a full step for every member.  Tiles of one member are
 // contiguous in the global order, and the XCD-aware block order keeps each
-// member's tiles together on one XCD where it can.
+// member's tiles together on one XCD where it can.  Hydro kernels are held to
+// the 168 VGPRs that three waves on a SIMD can have: the smaller tiles share a
+// CU, and stage 3 would take five more and lose a third of its waves.
 template <int TY, int STAGE, bool MAG, int TW>
-__global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_stage_ens(
+__global__ __launch_bounds__((TileShape<TY, TW>::NW * 64), MAG ? 2 : 3) void k_stage_ens(
     const EnsMember* __restrict__ mem, int nmem, int ntiles, int cur) {
     __shared__ StageLds<TY, STAGE, MAG, false, false, TW> lds;
     const int T = logical_block();
@@ -95,8 +104,8 @@ __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_stage_ens(
         if (mem[mid].tile0 <= T) lo = mid;
         else hi = mid - 1;
     }
-    const EnsMember& e = mem[lo];
-    member_tile<TY, STAGE, MAG, TW>(e, T - e.tile0, cur, lds);
+    const EnsTable m = (EnsTable)(mem + lo);
+    member_tile<TY, STAGE, MAG, TW>(m, T - m->tile0, cur, lds);
 }
 
 // Last member m with key(mem[m]) <= v (keys ascending from mem[0] = 0).
@@ -159,14 +168,15 @@ __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_ens_run(
                 __syncthreads();  // grab is rewritten by the next take
                 if (i >= n_x) break;
                 const int T = xcd * tiles_xcd + i;
-                const EnsMember& e =
-                    mem[find_member(mem, nmem, T, [](const EnsMember& x) { return x.tile0; })];
+                const EnsTable m = (EnsTable)(
+                    mem + find_member(mem, nmem, T, [](const EnsMember& x) { return x.tile0; }));
+                const int t = T - m->tile0;
                 if (s == 0)
-                    member_tile<TY, 0, MAG, TW>(e, T - e.tile0, cur, lds.s0);
+                    member_tile<TY, 0, MAG, TW>(m, t, cur, lds.s0);
                 else if (s == 1)
-                    member_tile<TY, 1, MAG, TW>(e, T - e.tile0, cur, lds.s1);
+                    member_tile<TY, 1, MAG, TW>(m, t, cur, lds.s1);
                 else
-                    member_tile<TY, 2, MAG, TW>(e, T - e.tile0, cur, lds.s2);
+                    member_tile<TY, 2, MAG, TW>(m, t, cur, lds.s2);
                 __syncthreads();  // the next tile reuses the LDS
             }
             base += n_x + per_xcd;
