@@ -37,6 +37,8 @@
 // the neighbour from the same operands, which yields the same doubles.
 #pragma once
 
+#include <type_traits>
+
 #include "r3d_dev.hpp"
 
 // The kernels live in namespace R3D_KNS: r3d for the bit-exact build; the
@@ -997,6 +999,14 @@ __device__ __forceinline__ void stage_walls(const StageArgs& a, const Consts& C,
     }
 }
 
+// k_stage's parameters as they lie in the kernel's argument segment: one after
+// another, each at its type's alignment, like the members of a struct.
+struct StageKernarg {
+    StageArgs a;
+    Consts C;
+    Metrics M;
+};
+
 // One RK stage of one run: block -> tile with the XCD-aware order.
 template <int TY, int STAGE, int ZMODE, bool MAG, bool HEAT = false, bool DEN = false, int TW = 64>
 __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_stage(const StageArgs a,
@@ -1008,19 +1018,23 @@ __global__ __launch_bounds__((TileShape<TY, TW>::NW * 64)) void k_stage(const St
     double pm[NPART];
     TileCell<TY, TW> me;
     if (stage_tile<TY, STAGE, ZMODE, MAG, HEAT, DEN, TW>(a, C, M, t, lds, pm, me)) {
-        struct Args {  // the arguments once more, from the kernel's argument segment
-            StageArgs a;
-            Consts C;
-            Metrics M;
-        };
-        auto* k =
-            (const __attribute__((address_space(4))) Args*)__builtin_amdgcn_kernarg_segment_ptr();
+        // the arguments once more, from the kernel's argument segment
+        auto* k = (const __attribute__((address_space(4)))
+                       StageKernarg*)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(k));
-        const Args& w = *(const Args*)k;
+        const StageKernarg& w = *(const StageKernarg*)k;
         stage_walls<TY, STAGE, ZMODE, MAG, TW>(w.a, w.C, w.M, me, pm);
     }
     if (STAGE == 2 && a.want_dt)
         block_partials<TileShape<TY, TW>::NW>(pm, lds.red, a.partial, t);
 }
+
+// What k_stage reads a second time is its parameter list.
+static_assert(std::is_same_v<decltype(&k_stage<8, 0, 0, false>),
+                             void (*)(StageArgs, Consts, Metrics)>,
+              "StageKernarg does not follow k_stage's parameters");
+static_assert(std::is_trivially_copyable_v<StageKernarg> &&
+                  sizeof(StageKernarg) == sizeof(StageArgs) + sizeof(Consts) + sizeof(Metrics),
+              "padding between k_stage's parameters");
 
 }  // namespace R3D_KNS
