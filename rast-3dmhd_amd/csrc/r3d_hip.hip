@@ -164,15 +164,15 @@ constexpr int hm_seg(int nch) { return nch == 1 ? 704 : 192; }
 template <int NCH, bool WW2>
 __global__ __launch_bounds__(hm_seg(NCH) + 64) void k_hmean_partial(const Geo g, const State x, int f,
                                                               const double* ttm, double* part,
-                                                              int npey, double cnt) {
+                                                              int npey, double cnt, int cus) {
     constexpr int HM_SEG = hm_seg(NCH);
     __shared__ __align__(16) double buf[2][NCH][HM_SEG + 2];
     const int chains = (g.npz + 2) * npey, nry = g.npy / npey;
     const int c0 = blockIdx.x * NCH, nc = min(NCH, chains - c0);
     const long len = (long)g.npx * nry;
     const int nseg = (int)((len + HM_SEG - 1) / HM_SEG);
-    // the summing wave: another one (another SIMD) in each round of blocks
-    const int wsum = (blockIdx.x >> 8) & 3, wave = threadIdx.x >> 6;
+    // the summing wave: another one (another SIMD) in each round of a block a CU
+    const int wsum = (blockIdx.x / cus) & 3, wave = threadIdx.x >> 6;
     if (wave == wsum) {
         const int c = threadIdx.x & 63;
         double sum = 0.0;
@@ -622,7 +622,7 @@ void launch_hmean_partial(r3d_hip_ctx* c, int f, const double* ttm) {
     const double cnt = (double)(p.npx * p.npy);
 #define R3D_HM(N, W)                                                                         \
     hipLaunchKernelGGL((k_hmean_partial<N, W>), dim3((chains + N - 1) / N), dim3(hm_seg(N) + 64), \
-                       0, c->stream, c->g, s, f, ttm, c->den_buf, p.npey, cnt)
+                       0, c->stream, c->g, s, f, ttm, c->den_buf, p.npey, cnt, c->cus)
     if (chains <= c->cus) {
         if (ttm) R3D_HM(1, true);
         else R3D_HM(1, false);
