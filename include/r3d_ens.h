@@ -5,7 +5,7 @@
  * Each RK stage of every member is one launch over a tile table spanning all
  * members; each member keeps its own dt (its own CFL reduction), scalars and
  * state, and its results are bit-identical to the same run stepped alone
- * through r3d_hip_step.  A full step (three stages, the boundary passes and
+ * through r3d_hip_step.  A full step (three stages with their boundary conditions,
  * the per-member dt reductions) is captured in a HIP graph and replayed.
  * Tile shapes are chosen by r3d_ens_autotune, which times the candidates on
  * the members themselves and restores their state afterwards.

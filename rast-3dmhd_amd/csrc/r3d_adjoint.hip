@@ -457,7 +457,7 @@ __device__ void dt_apply(const Geo& g, const State& X, const Consts& C, const Le
 // rest, say) all blocks go over the whole state, and the one that ends last
 // reduces their results.  The steps use the two slots in turn, so that a count
 // is cleared while no block can read it.  At 128x128x256 8 us a step (MHD 11),
-// and the bounds some 15 of the transpose's 230 (441); the pass over the state
+// and the bounds some 8 of the transpose's 224 (45 of 430); the pass over the state
 // took 41 (56) at the copy rate of the card, its reduction by one wave 16 more.
 __global__ __launch_bounds__(AT) void k_dt_adj(const Geo g, const State X, const Consts C,
                                                const Metrics M, const DtHits H, int* counts,

@@ -49,7 +49,7 @@ namespace r3d {
 // What plane p emits in z stays in the column's registers: plane p - 1 is
 // finished with it and stored, and plane p + 1 starts from it.
 //
-// At 128x128x256 a launch takes 217 us (MHD 382; 230 and 441 where it also lists
+// At 128x128x256 a launch takes 216 us (MHD 385; 224 and 430 where it also lists
 // the cells that may set dt), where the bytes it cannot do without (the state,
 // LA, LB and LO once each: 160 and 256 a cell) take 143 (229) at the copy rate of
 // the card; with two barriers a plane hydro took 226 (248).  Two waves per SIMD,
